@@ -192,8 +192,8 @@ def tile_phases(torch, ex, runs: int = 3) -> dict:
     over summed stages), the hand-over of the next index, the epilogue until its last wave is done,
     next_start: from the last epilogue wave's end to the same workgroup's next tile start
     (negative where its first waves start the next tile while the slowest still stores), and
-    middle_step: the per-wave parts of the k-loop step k = stages / 2.  The median launch of
-    `runs`."""
+    middle_step: the per-wave parts of the k-loop step k = stages / 2 (for tiles of the class whole,
+    whose step is four like phases, the cycles of each phase).  The median launch of `runs`."""
     import numpy as np
 
     from grouped_gemm_gpu_kernel_amd import _lib
@@ -260,6 +260,8 @@ def tile_phases(torch, ex, runs: int = 3) -> dict:
                         "wait": round(float(np.nanmean(parts[2]))), "barrier": round(float(np.nanmean(parts[3]))),
                         "barrier_max_wave": round(float(np.nanmean(np.nanmax(parts[3], axis=1)))),
                         "step": round(float(span.mean()))}
+            if name == "whole" and bm > 128:
+                step_row = {"phases": [round(float(np.nanmean(x))) for x in parts], "step": round(float(span.mean()))}
         out[name] = {
             "tiles": int(sel.sum()), "stages": round(float(stages[sel].mean()), 2),
             "first_stage": round(float((first - start)[sel].mean())),

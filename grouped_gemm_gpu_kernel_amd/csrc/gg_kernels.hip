@@ -364,22 +364,14 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
             args.tile_map[3 * ref + 2] = tn;
           }
         }
-      } else if (half == 0) {
-        if constexpr (TRACED) {
-          mark_tile_start<G>(stamps, 0, p, wm * G::BM, wn * G::BN);
-          run_work_tile<S, PATH, WIDE>(p, wm * G::BM, wn * G::BN, lds, request, after_k_loop, stamps);
-        } else {
-          run_work_tile<S, PATH, WIDE>(p, wm * G::BM, wn * G::BN, lds, request, after_k_loop);
-        }
       } else {
-        // One half of the rows (whole rows of macro-tiles), computed as a
+        // One half of the rows (whole rows of macro-tiles) is computed as a
         // problem that ends with that half: its tile has at most BM / 2 rows
         // and runs in a half-height edge class, and each of its D elements is
         // computed as in the whole tile.
         gg_device_problem_desc q = p;
-        const int m0 = wm * G::BM + (half - 1) * (G::BM / 2);
-        const int end = m0 + G::BM / 2;
-        q.m = end < p.m ? end : p.m;
+        const int m0 = wm * G::BM + (half == 2 ? G::BM / 2 : 0);
+        if (half != 0 && m0 + G::BM / 2 < p.m) q.m = m0 + G::BM / 2;
         if constexpr (TRACED) {
           mark_tile_start<G>(stamps, half, q, m0, wn * G::BN);
           run_work_tile<S, PATH, WIDE>(q, m0, wn * G::BN, lds, request, after_k_loop, stamps);

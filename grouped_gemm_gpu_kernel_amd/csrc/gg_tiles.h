@@ -9,6 +9,7 @@
 #pragma once
 
 #include "gg_common.h"
+#include "gg_phased.h"
 
 namespace gg {
 
@@ -155,6 +156,8 @@ struct MfmaTile {
   static constexpr int WN = G::BN / WAVES_N;
   static constexpr int FM = WM / 32;
   static constexpr int FN = WN / 32;
+  // The full 256 x 256 work tile in 128 x 64 wave blocks.
+  static constexpr bool PHASED = G::BM == 256 && G::BN == 256 && G::BK == 64 && G::THREADS == 512 && WM == 128;
   static_assert(WAVES_M * WAVES_N * kWave == G::THREADS, "one wave per block of D");
   static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile must hold whole 32x32 blocks");
   // 32-row groups of D per epilogue chunk: the whole block for blocks of up
@@ -253,6 +256,8 @@ struct MfmaTile {
     };
     if constexpr (WIDE) {
       run_k_loop<G, WIDE>(p, m0, n0, lds, compute, on_start, stamps);
+    } else if constexpr (PHASED) {
+      run_k_loop_phased<G>(p, m0, n0, lds, wm, wn, acc, on_start, stamps);
     } else {
       run_k_loop_dma<G>(p, m0, n0, lds, compute, on_start, stamps);
     }

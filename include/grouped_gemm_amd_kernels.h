@@ -256,7 +256,10 @@ enum {
   /* Entry GGK_PHASE_STEP + GGK_PHASE_STEP_MARKS w + i: wave w's core clock in the k-loop step
    * k = stages / 2 (LDS-DMA k-loops only; zero elsewhere): i = 0 the step starts, 1 its loads of
    * the next stage are issued, 2 its MFMAs and fragment reads are issued, 3 its loads have landed
-   * (the step's vmcnt wait is over), 4 the step's closing barrier is passed. */
+   * (the step's vmcnt wait is over), 4 the step's closing barrier is passed.  A work tile with more
+   * than half the rows and half the columns of a 256 x 256 one runs its step in four phases, each
+   * a quarter of the MFMAs, the loads and the fragment reads: there i = 1..4 is the end of phase
+   * i - 1. */
   GGK_PHASE_STEP = 8,
   GGK_PHASE_STEP_MARKS = 5,
   GGK_PHASE_STEP_WAVES = 8,   /* waves per workgroup at most */
