@@ -38,9 +38,10 @@ constexpr int kWave = 64;
 //   B: BK rows of BN values, row-major as in global memory, with the 8-byte
 //      chunks of row k stored at chunk index (c ^ b_swizzle(k)).  The
 //      transposing operand read touches 4 consecutive rows x 16 columns per
-//      16 lanes; the swizzle spreads those rows over disjoint banks without
-//      padding.  It flips only chunk-index bits >= 3, so 16-byte pieces
-//      (2 chunks) stay contiguous and every 32-column block stays intact.
+//      16 lanes, and the next 16 lanes the rows 8 further on; the swizzle
+//      spreads those 8 row pieces of 32 bytes over the 64 banks without
+//      padding.  It flips only chunk-index bits >= 2, so 16-byte pieces
+//      (2 chunks) stay contiguous and every 16-column block stays intact.
 //
 // Register staging: DEPTH stages are in flight in registers at once, the
 // loads of stage k + DEPTH - 1 issued while stage k is multiplied (a ring of
@@ -81,12 +82,14 @@ struct Geometry {
 
   // 64 banks x 4 bytes hold 256 bytes: two 64-column rows or half of a
   // 256-column row.  XOR-ing the chunk index with 8 moves a chunk by 64 bytes,
-  // so rows k..k+3 (k a multiple of 4) land on 4 different 64-byte bank windows.
+  // so rows k..k+3 (k a multiple of 4) land on 4 different 64-byte bank
+  // windows, and with 4 by 32 bytes, so rows k and k + 8 take different halves
+  // of a window.
   __device__ static __forceinline__ int b_swizzle(int k) {
     if constexpr (BN == 64) {
       return 8 * ((k >> 1) & 1);
     } else {
-      return 8 * (k & 3);
+      return 8 * (k & 3) + 4 * ((k >> 3) & 1);
     }
   }
   // Element offset, within a B stage, of the 4-value chunk that holds (k, n)
@@ -188,7 +191,7 @@ template <int V> struct KernelShape<V, GGK_PATH_MFMA> {
   // (four) LDS buffers fit -- two (three) stages in flight instead of one,
   // which is what a tile that streams its operands from HBM is bound by.  The
   // same 512 threads compute it in 64 x 64 (32 x 64) wave blocks; every D
-  // element is still one lane's 32x32x16 MFMA chain over ascending k with the
+  // element is still one lane's 16x16x32 MFMA chain over ascending k with the
   // same epilogue, so D does not depend on the class.
   static constexpr bool CLASSES = GG_TILE_CLASSES != 0 && kLarge && BM == 256 && BN == 256 && THREADS == 512;
   using GR = Geometry<BM / 2, BN, GG_STAGE_K, 2, THREADS, 3, true>;       // rows <= BM / 2
@@ -423,10 +426,10 @@ struct StageLoader<G, false> {
   static constexpr int APR = G::BK / 8;  // A pieces per row
   static constexpr int BPR = G::BN / 8;  // B pieces per k-row
   // LDS distance between a thread's consecutive pieces.  The B swizzle
-  // repeats every 4 k-rows, so it is the same for all of a thread's pieces.
+  // repeats every 16 k-rows, so it is the same for all of a thread's pieces.
   static constexpr int A_LDS_STEP = (T / APR) * G::SA;
   static constexpr int B_LDS_STEP = (T / BPR) * G::SB;
-  static_assert((T / BPR) % 4 == 0, "a thread's B pieces must share their swizzle");
+  static_assert((T / BPR) % 16 == 0, "a thread's B pieces must share their swizzle");
   static_assert(!G::A_SWIZZLED || (T / APR) % (G::A_RPW * APR) == 0, "a thread's A pieces must share their swizzle");
 
   const gg_device_problem_desc& p;
@@ -620,7 +623,7 @@ struct DmaLoader {
   static constexpr int APR = G::APR;     // A pieces per row
   static constexpr int BPR = G::BN / 8;  // B pieces per k-row
   static_assert((kWave * WAVES / APR) % (G::A_RPW * APR) == 0, "a thread's A pieces must share their swizzle");
-  static_assert((kWave * WAVES / BPR) % 4 == 0, "a thread's B pieces must share their swizzle");
+  static_assert((kWave * WAVES / BPR) % 16 == 0, "a thread's B pieces must share their swizzle");
   static constexpr int A_ROWS_STEP = kWave * WAVES / APR;  // rows between a thread's A pieces
   static constexpr int B_ROWS_STEP = kWave * WAVES / BPR;  // k-rows between a thread's B pieces
   static constexpr int LOADS = NA + NB;                    // load instructions per stage and wave

@@ -6,11 +6,11 @@
 // that use them.  With whole stages (all loads of the next stage issued at the
 // top of a step, one stage in flight) the waves spent a third of a step blocked
 // on issuing loads and as much waiting for them: a stage took 4,030 cycles
-// where its MFMAs need 2,048; here it takes 2,550 - 2,610.  One 8192^3 problem
-// 986 -> 872 us (1261 TFLOP/s), 64 x 2048^3 1217 -> 1059 us.  On random data
-// the clock falls to about 1.6 GHz under the chip's power limit (zeros: 591 us
-// at 2.4 GHz), so what bounds the loop now is energy per product first and the
-// 64 KB per stage from L2 (2,300 cycles without the MFMAs) next.
+// where its MFMAs need 2,048; here it takes 2,900 traced.  Same card: 64 x 2048^3
+// 1221 -> 1005 us, one 8192^3 problem 991 -> 814 us (1350 TFLOP/s).  On random
+// data the clock falls to 1.9 GHz and below under the chip's power limit (zeros:
+// 609 us at 2.4 GHz), so what bounds the loop is energy per product: without
+// its loads it takes 16% less time, without its fragment reads 17%.
 #pragma once
 
 #include <type_traits>
@@ -43,14 +43,15 @@ __device__ __forceinline__ void phase_barrier() {
 // is asked for once.  LDS holds two stages, [parity][A0, B0, B1, A1].
 //
 // A phase multiplies one pair (A half i, B half j): 64 rows x 64 columns x 32
-// deep per wave, 8 MFMAs.  The pairs follow (0,0), (0,1), (1,0), (1,1), so
+// deep per wave, 16 MFMAs.  The pairs follow (0,0), (0,1), (1,0), (1,1), so
 // every accumulator meets k in ascending order and a fragment read from LDS
 // serves two phases.  Phase f reads the fragments of unit f + 2 into
 // registers nothing uses any more (phases 0..3 of stage t: B1 of t, A1 of t,
 // A0 of t + 1, B0 of t + 1) and issues the loads of unit f + 8, into the slot
 // whose fragments were read in phase f - 2.  Its end waits until this wave's
 // loads of unit f + 3 have landed (five units stay in flight) and until its
-// own LDS reads are done; one barrier then tells every wave both.
+// LDS reads of the phases before have returned (a phase makes eight); one
+// barrier then tells every wave both.
 template <class G>
 struct PhasedLoader {
   static constexpr int UNIT = 128 * 64;  // values of a unit
@@ -160,7 +161,7 @@ struct PhasedLoader {
 // k-loops.
 template <class G, class OnStart, class Stamps>
 __device__ __forceinline__ void run_k_loop_phased(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds, int wm,
-                                                  int wn, floatx16_t (&acc)[4][2], OnStart&& on_start,
+                                                  int wn, floatx4_t (&acc)[8][4], OnStart&& on_start,
                                                   const Stamps& stamps) {
   using L = PhasedLoader<G>;
   const int nk = (p.k + G::BK - 1) / G::BK;
@@ -170,46 +171,51 @@ __device__ __forceinline__ void run_k_loop_phased(const gg_device_problem_desc& 
   }
   const L loader(p, m0, n0);
 
-  half8_t a[2][2][4];  // [A half][32-row block][16-deep k-step]
-  half8_t b[2][2][2];  // [B half][32-column block][k-step]
+  half8_t a[2][4][2];  // [A half][16-row block][32-deep k-step]
+  half8_t b[2][4];     // [B half, one k-step][16-column block]
   const int lane = opaque_tid() & (kWave - 1);
   const int g = lane >> 4, j = lane & 15;
-  // LDS byte address of the lane's fragment in the first units: block 0, k-step 0.
-  const uint32_t a_lane = lds_address(lds) + 2u * (uint32_t)G::a_piece(wm * 64 + (lane & 31), lane >> 5);
+  // LDS byte address of the lane's fragment in the first units: block 0, k-step 0
+  // (operand layouts as in MfmaTile).
+  const uint32_t a_lane = lds_address(lds) + 2u * (uint32_t)G::a_piece(wm * 64 + j, g);
   const uint32_t b_lane =
-      lds_address(lds) + 2u * (uint32_t)G::b_chunk(8 * (g >> 1) + (j >> 2), wn * 64 + 16 * (g & 1) + 4 * (j & 3));
+      lds_address(lds) + 2u * (uint32_t)G::b_chunk(8 * g + (j >> 2), wn * 64 + 4 * (j & 3));
 
   // Fragment read r (0..7) of the unit at offset `unit` (values) of a stage at
-  // byte offset `stage` of the ring.  The k-step selects bits 5 and 6 of A's
-  // address, the column block bit 6 of B's (the swizzles are XORs).
+  // byte offset `stage` of the ring.  The k-step selects bit 6 of A's address,
+  // the column block bits 5 and 6 of B's (the swizzles are XORs).
   auto read_a = [&](int half, int unit, uint32_t stage, int r) {
-    const int fm = r & 1, s = r >> 1;
-    const uint32_t at = (a_lane + stage) ^ (uint32_t)(32 * s);
-    a[half][fm][s] = *(const GG_LDS half8_t*)(uintptr_t)(at + 2u * (uint32_t)(unit + fm * 32 * G::SA));
+    const int fm = r & 3, s = r >> 2;
+    const uint32_t at = (a_lane + stage) ^ (uint32_t)(64 * s);
+    a[half][fm][s] = *(const GG_LDS half8_t*)(uintptr_t)(at + 2u * (uint32_t)(unit + fm * 16 * G::SA));
   };
   short4_t b_lo;
   auto read_b = [&](int half, int unit, uint32_t stage, int r) {
-    const int s = r >> 2, fn = (r >> 1) & 1;
-    const uint32_t at = ((b_lane + stage) ^ (uint32_t)(64 * fn)) + 2u * (uint32_t)(unit + s * 16 * G::SB);
+    const int fn = r >> 1;
+    const uint32_t at = ((b_lane + stage) ^ (uint32_t)(32 * fn)) + 2u * (uint32_t)unit;
     if ((r & 1) == 0) {
       b_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GG_LDS short4_t*)(uintptr_t)at);
     } else {
       const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GG_LDS short4_t*)(uintptr_t)(at + 8u * G::SB));
-      b[half][fn][s] = __builtin_bit_cast(half8_t, __builtin_shufflevector(b_lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      b[half][fn] = __builtin_bit_cast(half8_t, __builtin_shufflevector(b_lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
   };
-  // The 8 MFMAs of (A half, B half), each followed by read(r) of a later
-  // unit; issue(0) and issue(1) ask for the two loads of a unit later still.
+  // The 16 MFMAs of (A half, B half).  Each of the first 8 is followed by
+  // read(r) of a later unit, so that the fragments the next phase starts with
+  // have landed by then; issue(0) and issue(1) ask for the two loads of a unit
+  // later still, where no LDS read waits behind them (8192^3: 814 us; issued
+  // after MFMAs 3 and 9, 834; with the reads at every other MFMA, 834).
+  // Consecutive MFMAs share an operand: columns go back and forth.
   auto phase = [&](int ah, int bh, auto&& issue, auto&& read) {
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int s = r >> 2, fm = (r >> 1) & 1, fn = r & 1;
-      acc[2 * ah + fm][fn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ah][fm][2 * bh + s], b[bh][fn][s],
-                                                                     acc[2 * ah + fm][fn], 0, 0, 0);
+    for (int r = 0; r < 16; ++r) {
+      const int fm = r >> 2, fn = (fm & 1) != 0 ? 3 - (r & 3) : r & 3;
+      acc[4 * ah + fm][fn] =
+          __builtin_amdgcn_mfma_f32_16x16x32_f16(b[bh][fn], a[ah][fm][bh], acc[4 * ah + fm][fn], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-      read(r);
-      if (r == 1) issue(0);
-      if (r == 5) issue(1);
+      if (r < 8) read(r);
+      if (r == 8) issue(0);
+      if (r == 12) issue(1);
       __builtin_amdgcn_sched_barrier(0);
     }
     wait_lgkmcnt<8>();

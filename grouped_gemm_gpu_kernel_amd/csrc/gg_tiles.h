@@ -128,13 +128,21 @@ __device__ __forceinline__ void run_k_loop_dma(const gg_device_problem_desc& p, 
 }
 
 // ---------------------------------------------------------------------------
-// MFMA tile: v_mfma_f32_32x32x16_f16, (BM/WM) x (BN/WN) waves, each owning a
-// WM x WN block of D held as (WM/32) x (WN/32) 32x32 accumulators.
+// MFMA tile: v_mfma_f32_16x16x32_f16, (BM/WM) x (BN/64) waves, each owning a
+// WM x 64 block of D held as (WM/16) x 4 16x16 accumulators.  Per product the
+// 16x16x32 form reads and writes half the accumulators of the 32x32x16 one: on
+// random data, where the chip's power sets the clock, one 8192^3 problem took
+// 836 us with it against 873 us (though 630 against 590 us on zeros, where the
+// clock is at its limit).  Both give the same bits.
 //
-// Operand layouts of v_mfma_f32_32x32x16_f16 (lane l of 64):
-//   A: row l%32, k = 8*(l/32) + e, e = 0..7 (one 16-byte read of an A row)
-//   B: col l%32, k = 8*(l/32) + e
-//   D: acc[4*g + r] = D[8*g + 4*(l/32) + r][l%32], g, r = 0..3
+// D is computed transposed, with B as the instruction's first operand and A as
+// its second: a lane then holds 4 consecutive columns of one row of D, as the
+// epilogue reads C and writes D.
+//
+// Operand layouts of v_mfma_f32_16x16x32_f16 (lane l of 64):
+//   A: row l%16, k = 8*(l/16) + e, e = 0..7 (one 16-byte read of an A row)
+//   B: col l%16, k = 8*(l/16) + e
+//   D: acc[r] = D[l%16][4*(l/16) + r], r = 0..3
 // B sits in LDS row-major ([k][n]); ds_read_b64_tr_b16 turns four k-rows of
 // 16 columns into the k-contiguous operand.  Within each group of 16 lanes it
 // returns, to lane i, element i%4 of the 8-byte chunk addressed by lane
@@ -151,79 +159,59 @@ __device__ __forceinline__ void run_k_loop_dma(const gg_device_problem_desc& p, 
 template <class G, int WM_>
 struct MfmaTile {
   static constexpr int WM = WM_;
+  static constexpr int WN = 64;
   static constexpr int WAVES_M = G::BM / WM;
-  static constexpr int WAVES_N = G::THREADS / kWave / WAVES_M;
-  static constexpr int WN = G::BN / WAVES_N;
-  static constexpr int FM = WM / 32;
-  static constexpr int FN = WN / 32;
+  static constexpr int WAVES_N = G::BN / WN;
+  static constexpr int FM = WM / 16;
+  static constexpr int FN = WN / 16;
+  static_assert(WAVES_M * WAVES_N * kWave == G::THREADS, "one wave per block of D");
+  static_assert(WM % 32 == 0, "whole 16-row blocks, in pairs");
   // The full 256 x 256 work tile in 128 x 64 wave blocks.
   static constexpr bool PHASED = G::BM == 256 && G::BN == 256 && G::BK == 64 && G::THREADS == 512 && WM == 128;
-  static_assert(WAVES_M * WAVES_N * kWave == G::THREADS, "one wave per block of D");
-  static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile must hold whole 32x32 blocks");
-  // 32-row groups of D per epilogue chunk: the whole block for blocks of up
-  // to 2 x 2 accumulators (16 C vectors, 64 registers), one row of
-  // accumulators per chunk for larger blocks, which hold more registers.
-  static constexpr int EPI_ROWS = FM * FN <= 4 ? FM : 1;
-  static_assert(FM % EPI_ROWS == 0, "whole chunks");
+  // 16-row blocks of D per epilogue chunk: the whole block up to 64 rows (16 C
+  // vectors, 64 registers), 32 rows per chunk for larger blocks, which hold
+  // more registers.
+  static constexpr int EPI_BLOCKS = FM <= 4 ? FM : 2;
+  static_assert(FM % EPI_BLOCKS == 0, "whole chunks");
 
   // Multiplies one LDS stage into acc.  All MFMAs of a stage are issued
   // unconditionally; skipping is decided once per tile for the whole wave.
   __device__ __forceinline__ static void compute_stage(const uint16_t* stage, int lane, int wm, int wn,
-                                                       floatx16_t (&acc)[FM][FN]) {
+                                                       floatx4_t (&acc)[FM][FN]) {
     const uint16_t* as = stage;
     const uint16_t* bs = stage + G::A_STAGE;
     lane = opaque_tid() & (kWave - 1);
     const int g = lane >> 4;
     const int j = lane & 15;
-    // Operand fragments of k-step s (16 deep) of the stage.
+    // Operand fragments of k-step s (32 deep) of the stage.
     auto load_frags = [&](int s, half8_t (&af)[FM], half8_t (&bf)[FN]) {
 #pragma unroll
       for (int fm = 0; fm < FM; ++fm) {
-        const uint16_t* src = as + G::a_piece(wm * WM + fm * 32 + (lane & 31), 2 * s + (lane >> 5));
+        const uint16_t* src = as + G::a_piece(wm * WM + fm * 16 + j, 4 * s + g);
         af[fm] = *reinterpret_cast<const half8_t*>(src);
       }
 #pragma unroll
       for (int fn = 0; fn < FN; ++fn) {
-        const int nb = wn * WN + fn * 32 + 16 * (g & 1);
-        const int kb = s * 16 + 8 * (g >> 1);
-        // Rows kb + j/4 and kb + 4 + j/4 share one swizzle (it depends on k mod 4).
-        const uint16_t* src = bs + G::b_chunk(kb + (j >> 2), nb + 4 * (j & 3));
+        const int kb = s * 32 + 8 * g;
+        // Rows kb + j/4 and kb + 4 + j/4 share one swizzle.
+        const uint16_t* src = bs + G::b_chunk(kb + (j >> 2), wn * WN + fn * 16 + 4 * (j & 3));
         const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GG_LDS short4_t*)(src));
         const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GG_LDS short4_t*)(src + 4 * G::SB));
         bf[fn] = __builtin_bit_cast(half8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       }
     };
-    auto multiply = [&](const half8_t (&af)[FM], const half8_t (&bf)[FN]) {
+    constexpr int STEPS = G::BK / 32;
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      half8_t af[FM];
+      half8_t bf[FN];
+      load_frags(s, af, bf);
 #pragma unroll
       for (int fm = 0; fm < FM; ++fm) {
 #pragma unroll
         for (int fn = 0; fn < FN; ++fn) {
-          acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[fm], bf[fn], acc[fm][fn], 0, 0, 0);
+          acc[fm][fn] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[fn], af[fm], acc[fm][fn], 0, 0, 0);
         }
-      }
-    };
-    constexpr int STEPS = G::BK / 16;
-    if constexpr (FM * FN <= 4) {
-      // Small wave blocks: the compiler may schedule the whole stage freely.
-#pragma unroll
-      for (int s = 0; s < STEPS; ++s) {
-        half8_t af[FM];
-        half8_t bf[FN];
-        load_frags(s, af, bf);
-        multiply(af, bf);
-      }
-    } else {
-      // Large wave blocks: fragments of step s + 1 are read while step s is
-      // multiplied, and no further -- reading the whole stage ahead would
-      // need more registers than the accumulators leave.
-      half8_t af[2][FM];
-      half8_t bf[2][FN];
-      load_frags(0, af[0], bf[0]);
-#pragma unroll
-      for (int s = 0; s < STEPS; ++s) {
-        if (s + 1 < STEPS) load_frags(s + 1, af[(s + 1) & 1], bf[(s + 1) & 1]);
-        multiply(af[s & 1], bf[s & 1]);
-        __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
@@ -243,13 +231,11 @@ struct MfmaTile {
     // multiply or store; it still stages its share of A and B for the others.
     const bool live = m0 + wm * WM < p.m && n0 + wn * WN < p.n;
 
-    floatx16_t acc[FM][FN];
+    floatx4_t acc[FM][FN];
 #pragma unroll
     for (int fm = 0; fm < FM; ++fm)
 #pragma unroll
-      for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[fm][fn][e] = 0.0f;
+      for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     auto compute = [&](const uint16_t* stage) {
       if (live) compute_stage(stage, lane, wm, wn, acc);
@@ -270,116 +256,104 @@ struct MfmaTile {
   // 4 x 4 transpose across the 4 lanes of a quad: lane q holds x[k] = M[q][k]
   // and receives M[k][q], in two exchange steps (partner q^1, then q^2).
   __device__ __forceinline__ static void quad_transpose(float (&x)[4], int q) {
-    const bool odd = (q & 1) != 0;
-    const float s0 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(odd ? x[0] : x[1]), 0xB1, 0xf, 0xf, true));
-    const float s1 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(odd ? x[2] : x[3]), 0xB1, 0xf, 0xf, true));
-    float y[4];
-    y[0] = odd ? s0 : x[0];
-    y[1] = odd ? x[1] : s0;
-    y[2] = odd ? s1 : x[2];
-    y[3] = odd ? x[3] : s1;
-    const bool hi = (q & 2) != 0;
-    const float t0 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(hi ? y[0] : y[2]), 0x4E, 0xf, 0xf, true));
-    const float t1 = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(hi ? y[1] : y[3]), 0x4E, 0xf, 0xf, true));
-    x[0] = hi ? t0 : y[0];
-    x[1] = hi ? t1 : y[1];
-    x[2] = hi ? y[2] : t0;
-    x[3] = hi ? y[3] : t1;
+    const auto xor1 = [](float v) {
+      return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));
+    };
+    const auto xor2 = [](float v) {
+      return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true));
+    };
+    // Exchanged by every lane (a lane that is switched off would send zeros), then selected.
+    const float s0 = xor1(x[1]), s1 = xor1(x[0]), s2 = xor1(x[3]), s3 = xor1(x[2]);
+    const bool odd = (q & 1) != 0, high = (q & 2) != 0;
+    const float y0 = odd ? s0 : x[0];
+    const float y1 = odd ? x[1] : s1;
+    const float y2 = odd ? s2 : x[2];
+    const float y3 = odd ? x[3] : s3;
+    const float t0 = xor2(y2), t1 = xor2(y3), t2 = xor2(y0), t3 = xor2(y1);
+    x[0] = high ? t0 : y0;
+    x[1] = high ? t1 : y1;
+    x[2] = high ? y2 : t2;
+    x[3] = high ? y3 : t3;
   }
 
   // D = alpha * acc + beta * C for the wave's block at (r0, c0).
   //
-  // Accumulator element 4g + r of 32x32 block (fm, fn) is D[8g + 4h + r][c] of
-  // the block for lane (h, c) = (lane / 32, lane % 32).  A 4 x 4 transpose in
-  // each quad of lanes (c = 4j .. 4j+3) gives lane (h, 4j + q) row 8g + 4h + q,
-  // columns 4j .. 4j+3, so C is read and D written as 16-byte vectors: a
-  // dword access costs the address unit as much as a 16-byte one.
+  // Lane (g, j) = (lane / 16, lane % 16) holds, of 16x16 block (fm, fn), row
+  // 16 fm + j, columns 16 fn + 4 g .. + 3.  A 4 x 4 transpose in each quad of
+  // lanes (over fn, for each of the 4 columns) gives lane (g, 4 jj + q) the
+  // rows 16 fm + 4 jj + r, r = 0..3, columns 16 q + 4 g .. + 3: C is read and
+  // D written as 16-byte vectors (a dword access costs the address unit as
+  // much as a 16-byte one), and one access instruction covers 4 rows x 64
+  // columns, 256 contiguous bytes of each row.  Rows of tightly packed matrices
+  // (ldc = ldd = N) seldom start on a 128-byte line, and 256 contiguous bytes of
+  // such a row span 3 lines where four separate 64-byte pieces span 6.
   //
   // With 32-bit addressing C is read through a buffer resource from (r0, c0)
   // to the end of C: rows past M read as zero, so the loads need no branch.
-  // The block is written in chunks of EPI_ROWS 32-row groups, and all C
+  // The block is written in chunks of EPI_BLOCKS 16-row blocks, and all C
   // vectors of the next chunk (two, for blocks of three or more chunks) are
-  // requested before the current one is written, so their latencies overlap.  Stores go through the same kind of resource; columns that cross
-  // N go element by element.
-  // D = alpha * acc + beta * C for a wave block two 32-column blocks wide (FN == 2), written so
-  // that one 16-byte access instruction covers 4 rows x 64 columns (256 contiguous bytes of each
-  // row) instead of 8 rows x 32 columns.  After the quad transpose, lane (h, c) holds row
-  // 8g + 4h + (c & 3) of both column blocks; one v_permlane32_swap per value then gives every
-  // lane rows 8g + (c & 3) and 8g + 4 + (c & 3), lanes 0..31 of column block 0 and lanes 32..63
-  // of block 1.  Rows of tightly packed matrices (ldc = ldd = N) seldom start on a 128-byte line,
-  // and 256 contiguous bytes of such a row span 3 lines where two separate 128-byte pieces span
-  // 4: C reads and D writes make a quarter fewer L1 -> L2 requests.  Loading C, multiplying and
-  // storing follow store_tile (chunks of EPI_ROWS accumulator rows, the next chunks' C requested
-  // ahead).
-  __device__ __forceinline__ static void store_pairs(const gg_device_problem_desc& p, int r0, int c0, int lane,
-                                                     const floatx16_t (&acc)[FM][FN], bool use_c) {
-    static_assert(FN == 2, "two 32-column blocks");
-    const int q = lane & 3;
-    const int col = 32 * (lane >> 5) + ((lane & 31) & ~3);  // first of the lane's 4 columns in the block
-    const int ncol = p.n - (c0 + col);                        // how many of them lie inside the matrix
-    const __amdgpu_buffer_rsrc_t drs =
-        buffer_rsrc(p.d + ((int64_t)r0 * p.ldd + c0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldd + (p.n - c0)));
-    constexpr int CHUNKS = FM / EPI_ROWS;
-    constexpr int AHEAD = CHUNKS >= 3 ? GG_EPI_AHEAD : 1;
-    // C vectors of a chunk: [accumulator row][row group g][rows 8g + q, 8g + 4 + q].
-    floatx4_t cv[AHEAD + 1][EPI_ROWS][4][2];
-    auto load_c = [&](int chunk, floatx4_t (&dst)[EPI_ROWS][4][2]) {
-      if (use_c) {
-        const __amdgpu_buffer_rsrc_t crs =
-            buffer_rsrc(p.c + ((int64_t)r0 * p.ldc + c0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldc + (p.n - c0)));
+  // requested before the current one is written, so their latencies overlap.
+  // Stores go through the same kind of resource; columns that cross N go
+  // element by element.
+  template <bool WIDE>
+  __device__ __forceinline__ static void store_tile(const gg_device_problem_desc& p, int r0, int c0, int lane,
+                                                    const floatx4_t (&acc)[FM][FN]) {
+    const bool use_c = p.c != nullptr && p.beta != 0.0f;
+    if constexpr (!WIDE) {
+      const int q = lane & 3;
+      const int row_lane = 4 * ((lane >> 2) & 3);   // first of the lane's 4 rows in a 16-row block
+      const int col = 16 * q + 4 * (lane >> 4);     // first of its 4 columns in the wave block
+      const int ncol = p.n - (c0 + col);            // how many of them lie inside the matrix
+      const __amdgpu_buffer_rsrc_t drs =
+          buffer_rsrc(p.d + ((int64_t)r0 * p.ldd + c0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldd + (p.n - c0)));
+      constexpr int CHUNKS = FM / EPI_BLOCKS;
+      constexpr int AHEAD = CHUNKS >= 3 ? GG_EPI_AHEAD : 1;
+      floatx4_t cv[AHEAD + 1][EPI_BLOCKS][4];  // C vectors of a chunk: [16-row block][row of the lane]
+      auto load_c = [&](int chunk, floatx4_t (&dst)[EPI_BLOCKS][4]) {
+        if (use_c) {
+          const __amdgpu_buffer_rsrc_t crs =
+              buffer_rsrc(p.c + ((int64_t)r0 * p.ldc + c0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldc + (p.n - c0)));
 #pragma unroll
-        for (int i = 0; i < EPI_ROWS; ++i)
+          for (int i = 0; i < EPI_BLOCKS; ++i)
 #pragma unroll
-          for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int hf = 0; hf < 2; ++hf) {
-              const int row = (chunk * EPI_ROWS + i) * 32 + 8 * g + 4 * hf + q;
+            for (int r = 0; r < 4; ++r) {
+              const int row = (chunk * EPI_BLOCKS + i) * 16 + row_lane + r;
               // Vectors wholly past N would read the next row's head: an offset past the resource.
               const uint32_t off =
                   ncol > 0 ? 4u * ((uint32_t)row * (uint32_t)p.ldc + col) : DmaLoader<G>::kOutOfRange;
-              dst[i][g][hf] =
-                  __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(crs, (int)off, 0, 0));
+              dst[i][r] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(crs, (int)off, 0, 0));
             }
-      } else {
+        } else {
 #pragma unroll
-        for (int i = 0; i < EPI_ROWS; ++i)
+          for (int i = 0; i < EPI_BLOCKS; ++i)
 #pragma unroll
-          for (int g = 0; g < 4; ++g)
+            for (int r = 0; r < 4; ++r) dst[i][r] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+      };
 #pragma unroll
-            for (int hf = 0; hf < 2; ++hf) dst[i][g][hf] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int c = 0; c < AHEAD; ++c) {
+        if (c < CHUNKS) load_c(c, cv[c]);
       }
-    };
 #pragma unroll
-    for (int c = 0; c < AHEAD; ++c) {
-      if (c < CHUNKS) load_c(c, cv[c]);
-    }
+      for (int chunk = 0; chunk < CHUNKS; ++chunk) {
+        if (chunk + AHEAD < CHUNKS) load_c(chunk + AHEAD, cv[(chunk + AHEAD) % (AHEAD + 1)]);
 #pragma unroll
-    for (int chunk = 0; chunk < CHUNKS; ++chunk) {
-      if (chunk + AHEAD < CHUNKS) load_c(chunk + AHEAD, cv[(chunk + AHEAD) % (AHEAD + 1)]);
-#pragma unroll
-      for (int i = 0; i < EPI_ROWS; ++i) {
-        const int fm = chunk * EPI_ROWS + i;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          float v0[4] = {acc[fm][0][4 * g + 0], acc[fm][0][4 * g + 1], acc[fm][0][4 * g + 2], acc[fm][0][4 * g + 3]};
-          float v1[4] = {acc[fm][1][4 * g + 0], acc[fm][1][4 * g + 1], acc[fm][1][4 * g + 2], acc[fm][1][4 * g + 3]};
-          quad_transpose(v0, q);
-          quad_transpose(v1, q);
-          float vh[2][4];
+        for (int i = 0; i < EPI_BLOCKS; ++i) {
+          const int fm = chunk * EPI_BLOCKS + i;
+          float v[4][4];  // [column of the lane][row of the lane]
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v0[e]), __float_as_uint(v1[e]), false,
-                                                            false);
-            vh[0][e] = __uint_as_float(r[0]);
-            vh[1][e] = __uint_as_float(r[1]);
+#pragma unroll
+            for (int fn = 0; fn < 4; ++fn) v[e][fn] = acc[fm][fn][e];
+            quad_transpose(v[e], q);
           }
 #pragma unroll
-          for (int hf = 0; hf < 2; ++hf) {
-            const int row = fm * 32 + 8 * g + 4 * hf + q;
+          for (int r = 0; r < 4; ++r) {
+            const int row = fm * 16 + row_lane + r;
             floatx4_t out;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              out[e] = epilogue_value(vh[hf][e], cv[chunk % (AHEAD + 1)][i][g][hf][e], p.alpha, use_c ? p.beta : 0.0f);
+              out[e] = epilogue_value(v[e][r], cv[chunk % (AHEAD + 1)][i][r][e], p.alpha, use_c ? p.beta : 0.0f);
             }
             if (r0 + row >= p.m || ncol <= 0) continue;
             const uint32_t off = 4u * ((uint32_t)row * (uint32_t)p.ldd + col);
@@ -394,93 +368,6 @@ struct MfmaTile {
             }
           }
         }
-      }
-      // Keep each chunk's loads and stores in place (see store_tile).
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-
-  template <bool WIDE>
-  __device__ __forceinline__ static void store_tile(const gg_device_problem_desc& p, int r0, int c0, int lane,
-                                                    const floatx16_t (&acc)[FM][FN]) {
-    const bool use_c = p.c != nullptr && p.beta != 0.0f;
-    const int q = lane & 3;
-    const int lrow = 4 * (lane >> 5) + q;  // row within an 8-row group
-    const int lcol = (lane & 31) & ~3;     // first column of the lane's vector
-    if constexpr (!WIDE && FN == 2) {
-      store_pairs(p, r0, c0, lane, acc, use_c);
-    } else if constexpr (!WIDE) {
-      const __amdgpu_buffer_rsrc_t drs =
-          buffer_rsrc(p.d + ((int64_t)r0 * p.ldd + c0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldd + (p.n - c0)));
-      // C vectors of EPI_ROWS 32-row groups per chunk; the C of the next
-      // AHEAD chunks is requested before the current chunk is stored.
-      constexpr int CHUNKS = FM / EPI_ROWS;
-      constexpr int AHEAD = CHUNKS >= 3 ? GG_EPI_AHEAD : 1;  // chunks of C requested ahead
-      floatx4_t cv[AHEAD + 1][EPI_ROWS][FN][4];
-      auto load_c = [&](int chunk, floatx4_t (&dst)[EPI_ROWS][FN][4]) {
-        if (use_c) {
-          const __amdgpu_buffer_rsrc_t crs =
-              buffer_rsrc(p.c + ((int64_t)r0 * p.ldc + c0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldc + (p.n - c0)));
-#pragma unroll
-          for (int i = 0; i < EPI_ROWS; ++i)
-#pragma unroll
-            for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-              for (int g = 0; g < 4; ++g) {
-                const int fm = chunk * EPI_ROWS + i;
-                // Vectors wholly past N would read the next row's head (inside
-                // the resource) for nothing: they take an offset past it.
-                const bool in_n = c0 + fn * 32 + lcol < p.n;
-                const uint32_t off =
-                    in_n ? 4u * ((uint32_t)(fm * 32 + 8 * g + lrow) * (uint32_t)p.ldc + fn * 32 + lcol)
-                         : DmaLoader<G>::kOutOfRange;
-                dst[i][fn][g] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(crs, (int)off, 0, 0));
-              }
-        } else {
-#pragma unroll
-          for (int i = 0; i < EPI_ROWS; ++i)
-#pragma unroll
-            for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-              for (int g = 0; g < 4; ++g) dst[i][fn][g] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-      };
-#pragma unroll
-      for (int c = 0; c < AHEAD; ++c) {
-        if (c < CHUNKS) load_c(c, cv[c]);
-      }
-#pragma unroll
-      for (int chunk = 0; chunk < CHUNKS; ++chunk) {
-        if (chunk + AHEAD < CHUNKS) load_c(chunk + AHEAD, cv[(chunk + AHEAD) % (AHEAD + 1)]);
-#pragma unroll
-        for (int i = 0; i < EPI_ROWS; ++i) {
-          const int fm = chunk * EPI_ROWS + i;
-#pragma unroll
-          for (int fn = 0; fn < FN; ++fn) {
-            const int ncol = p.n - (c0 + fn * 32 + lcol);  // columns of the vector inside the matrix
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              float v[4] = {acc[fm][fn][4 * g + 0], acc[fm][fn][4 * g + 1], acc[fm][fn][4 * g + 2],
-                            acc[fm][fn][4 * g + 3]};
-              quad_transpose(v, q);
-              const int rrow = fm * 32 + 8 * g + lrow;
-              floatx4_t out;
-#pragma unroll
-              for (int e = 0; e < 4; ++e) out[e] = epilogue_value(v[e], cv[chunk % (AHEAD + 1)][i][fn][g][e], p.alpha, use_c ? p.beta : 0.0f);
-              if (r0 + rrow >= p.m || ncol <= 0) continue;
-              const uint32_t off = 4u * ((uint32_t)rrow * (uint32_t)p.ldd + fn * 32 + lcol);
-              if (ncol >= 4) {
-                __builtin_amdgcn_raw_buffer_store_b128(
-                    __builtin_bit_cast(__attribute__((ext_vector_type(4))) int, out), drs, (int)off, 0, 0);
-              } else {
-#pragma unroll
-                for (int e = 0; e < 3; ++e) {
-                  if (e < ncol) __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(out[e]), drs, (int)(off + 4 * e), 0, 0);
-                }
-              }
-            }
-          }
-        }
         // Keep each chunk's loads and stores in place: hoisting every C load
         // to the top would hold the whole block's C in registers.
         __builtin_amdgcn_sched_barrier(0);
@@ -488,22 +375,18 @@ struct MfmaTile {
     } else {
 #pragma unroll
       for (int fm = 0; fm < FM; ++fm) {
+        const int row = r0 + fm * 16 + (lane & 15);
 #pragma unroll
         for (int fn = 0; fn < FN; ++fn) {
-          const int col = c0 + fn * 32 + lcol;
+          const int col = c0 + fn * 16 + 4 * (lane >> 4);
           const int ncol = p.n - col;
+          if (row >= p.m || ncol <= 0) continue;
+          g_cf32_t* crow = (g_cf32_t*)p.c + ((int64_t)row * p.ldc + col);
+          g_f32_t* drow = (g_f32_t*)p.d + ((int64_t)row * p.ldd + col);
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            float v[4] = {acc[fm][fn][4 * g + 0], acc[fm][fn][4 * g + 1], acc[fm][fn][4 * g + 2],
-                          acc[fm][fn][4 * g + 3]};
-            quad_transpose(v, q);
-            const int row = r0 + fm * 32 + 8 * g + lrow;
-            if (row >= p.m || ncol <= 0) continue;
-            g_cf32_t* crow = (g_cf32_t*)p.c + ((int64_t)row * p.ldc + col);
-            g_f32_t* drow = (g_f32_t*)p.d + ((int64_t)row * p.ldd + col);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              if (e < ncol) drow[e] = epilogue_value(v[e], use_c ? crow[e] : 0.0f, p.alpha, use_c ? p.beta : 0.0f);
+          for (int e = 0; e < 4; ++e) {
+            if (e < ncol) {
+              drow[e] = epilogue_value(acc[fm][fn][e], use_c ? crow[e] : 0.0f, p.alpha, use_c ? p.beta : 0.0f);
             }
           }
         }
