@@ -689,25 +689,25 @@ struct DmaLoader {
     return (uint32_t)(bytes < 0 ? 0 : (bytes > (int64_t)kOutOfRange ? (int64_t)kOutOfRange : bytes));
   }
 
-  // Issues the loads of stage kt into LDS buffer `stage` (a stage's first element).
-  __device__ __forceinline__ void issue(int kt, uint16_t* stage) const {
+  // Issues load `l` (of LOADS: A's first) of stage kt into LDS buffer `stage` (a stage's first
+  // element).
+  __device__ __forceinline__ void issue_load(int kt, uint16_t* stage, int l) const {
     const uint32_t base = lds_address(stage) + 2u * (uint32_t)(wave * kWave * 8);
-    const uint32_t a_n = records(a_bytes);
-    // A pieces that start at k >= K are zero in the product; they are not
-    // fetched (the piece that straddles K is, and is repaired afterwards).
-    const uint32_t a_voff = kt * G::BK + 8 * a_col8 < k ? a_off : kOutOfRange;
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      load_to_lds16(a_tile, a_n, base + 2u * (uint32_t)(i * WAVES * kWave * 8), a_voff,
-                    2u * G::BK * (uint32_t)kt + i * a_step);
+    if (l < NA) {
+      // A pieces that start at k >= K are zero in the product; they are not
+      // fetched (the piece that straddles K is, and is repaired afterwards).
+      const uint32_t a_voff = kt * G::BK + 8 * a_col8 < k ? a_off : kOutOfRange;
+      load_to_lds16(a_tile, records(a_bytes), base + 2u * (uint32_t)(l * WAVES * kWave * 8), a_voff,
+                    2u * G::BK * (uint32_t)kt + l * a_step);
+    } else {
+      const int64_t skip = 2 * (int64_t)G::BK * kt * ldb;
+      load_to_lds16(b_tile + skip / 2, records(b_bytes - skip),
+                    base + 2u * (uint32_t)(G::A_STAGE + (l - NA) * WAVES * kWave * 8), b_off, (l - NA) * b_step);
     }
-    const int64_t skip = 2 * (int64_t)G::BK * kt * ldb;
-    const uint32_t b_n = records(b_bytes - skip);
+  }
+  __device__ __forceinline__ void issue(int kt, uint16_t* stage) const {
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      load_to_lds16(b_tile + skip / 2, b_n, base + 2u * (uint32_t)(G::A_STAGE + i * WAVES * kWave * 8), b_off,
-                    i * b_step);
-    }
+    for (int l = 0; l < LOADS; ++l) issue_load(kt, stage, l);
   }
 
   // Repairs this thread's pieces of stage kt (the one that holds k = K - 1)

@@ -1,9 +1,12 @@
 // gg_tiles.h -- macro-tile compute for the gfx950 grouped GEMM.
 //
-// Both tile paths share one pipeline: each K stage is read from global memory
-// into registers while the previous stage, held in LDS, is being multiplied;
-// the registers are then written to the other LDS buffer and one barrier ends
-// the stage.  The reference's equivalents are compute_gemm_tile_tensor_core and
+// The MFMA path loads its stages straight into LDS and multiplies them a phase
+// behind the fragment reads (run_k_loop_halves here, run_k_loop_phased in
+// gg_phased.h for the full 256 x 256 work tile).  The FMA path and the 64-bit
+// addressing forms stage through registers: each K stage is read from global
+// memory into registers while the previous stage, held in LDS, is being
+// multiplied; the registers are then written to the other LDS buffer and one
+// barrier ends the stage.  The reference's equivalents are compute_gemm_tile_tensor_core and
 // compute_gemm_tile_simt (src/grouped_gemm.cu:373-626); the k-loop structure,
 // register blocking and LDS layout here are gfx950's own.
 #pragma once
@@ -66,65 +69,178 @@ __device__ __forceinline__ void run_k_loop(const gg_device_problem_desc& p, int 
   }
 }
 
-// The k-loop with stage loads straight into LDS (32-bit offsets): BUFFERS
-// LDS buffers, BUFFERS - 1 stages in flight.  While stage k is multiplied out
-// of buffer k % BUFFERS, the loads of stage k + BUFFERS - 1 go to the buffer
-// every wave finished multiplying in the previous step; each wave then waits
-// until its own loads of stage k + 1 have landed (the stage holding K - 1 is
-// repaired then), and a barrier without a memory fence closes the step -- a
-// fenced barrier would also wait for the stages still in flight.  Loads are
-// issued for stages past K too (they read as zero or land unread).
+// The k-loop with stage loads straight into LDS (32-bit offsets) of wave
+// blocks of up to 64 x 64, BUFFERS LDS buffers of one stage each.
 //
-// on_start runs in the first step, after the loads of stage L are issued: a
-// request it makes is then the youngest in flight, and the first step's wait
-// lets it stay in flight (loads complete in order, so one more outstanding
-// operation is exactly that request).  The second step's wait retires it, so
-// it has two stage computations to come back.
-template <class G, class Compute, class OnStart, class Stamps>
-__device__ __forceinline__ void run_k_loop_dma(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
-                                               Compute&& compute, OnStart&& on_start, const Stamps& stamps) {
+// A stage is multiplied in two phases, its k-halves (32 deep, FM x 4 MFMAs per
+// wave); each phase reads the fragments of the next half into the registers
+// the phase before used, so no MFMA waits for a read that was issued just
+// before it.  The second half's fragments are read in phase 0, so a stage's
+// buffer is free from phase 1 on: the loads of stage t + BUFFERS go there in
+// phase 1 of stage t and (where more than one stage stays in flight) phase 0
+// of stage t + 1.  One wait and one barrier per stage, at the end of phase 0:
+// the wave's loads of stage t + 1 have landed (the stage holding K - 1 is
+// repaired then), and its reads of stage t are done.
+//
+// Stages past K are never asked for: a problem of fewer stages than BUFFERS
+// issues what it has and waits for all of it.
+//
+// These tiles are bound by latency and by what they stream rather than by the
+// matrix cores.  Against whole stages read and multiplied in one go, same
+// card: a 24-problem ragged set (half of it edge classes) 168.5 -> 146.9 us, 16
+// problems of at most 256 in each dimension 14.0 -> 12.7, mixed-512 222.9 ->
+// 220.5.
+//
+// on_start runs after the first barrier: the request it makes is then the
+// youngest operation in flight, and the first stage's wait lets it stay there.
+template <class G, int WM, class OnStart, class Stamps>
+__device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds, int wm,
+                                                  int wn, floatx4_t (&acc)[WM / 16][4], OnStart&& on_start,
+                                                  const Stamps& stamps) {
+  using L = DmaLoader<G>;
   constexpr int NBUF = G::BUFFERS;
-  constexpr int L = NBUF - 1;
-  constexpr int PENDING = (L - 1) * DmaLoader<G>::LOADS;  // loads of later stages allowed in flight
+  constexpr int FM = WM / 16;
+  constexpr int LOADS = L::LOADS;
+  // Loads of a stage issued in phase 1; the rest follow in the next phase 0.
+  constexpr int FIRST = NBUF > 2 ? LOADS / 2 : LOADS;
   const int nk = (p.k + G::BK - 1) / G::BK;
   if (nk <= 0) {
     on_start();
     return;
   }
-  const DmaLoader<G> loader(p, m0, n0);
+  const L loader(p, m0, n0);
+  const bool deep = nk >= NBUF;  // every buffer gets a stage
 #pragma unroll
-  for (int s = 0; s < L; ++s) loader.issue(s, lds + s * G::STAGE);
-  wait_vmcnt<PENDING>();
+  for (int s = 0; s < NBUF - 1; ++s) {
+    if (s < nk) loader.issue(s, lds + s * G::STAGE);
+  }
+  if (deep) {
+#pragma unroll
+    for (int l = 0; l < FIRST; ++l) loader.issue_load(NBUF - 1, lds + (NBUF - 1) * G::STAGE, l);
+    wait_vmcnt<(NBUF - 2) * LOADS + FIRST>();
+  } else {
+    wait_vmcnt<0>();
+  }
   stamps.mark(GGK_PHASE_FIRST_STAGE);
   if (loader.last_stage == 0) loader.fix_last_stage(0, lds);
   stage_barrier();
   stamps.mark(GGK_PHASE_K_LOOP);
-  // One step per iteration, not unrolled: no register set has to be indexed
-  // statically, and one copy of the step keeps the code a launch has to fetch
-  // into a cold instruction cache small.  u is the buffer of stage k.
-  int u = 0;
-#pragma unroll 1
-  for (int k = 0; k < nk; ++k) {
-    const int ul = u == 0 ? L : u - 1;  // (u + L) % NBUF
-    const int un = u == NBUF - 1 ? 0 : u + 1;
-    const bool stamped = k == nk / 2;  // the step whose timing a traced launch records
-    if (stamped) stamps.step_mark(0);
-    loader.issue(k + L, lds + ul * G::STAGE);
-    const bool extra = k == 0 && __builtin_amdgcn_readfirstlane(on_start() ? 1 : 0) != 0;
-    if (stamped) stamps.step_mark(1);
-    compute(lds + u * G::STAGE);
-    if (stamped) stamps.step_mark(2);
-    if (extra) {
-      wait_vmcnt<PENDING + 1>();
+  const bool extra = __builtin_amdgcn_readfirstlane(on_start() ? 1 : 0) != 0;
+
+  half8_t a[2][FM];  // [k-half][16-row block]
+  half8_t b[2][4];   // [k-half][16-column block]
+  const int lane = opaque_tid() & (kWave - 1);
+  const int g = lane >> 4, j = lane & 15;
+  // LDS byte address of the lane's fragments of block 0, k-half 0 (operand layouts as in MfmaTile).
+  const uint32_t a_lane = lds_address(lds) + 2u * (uint32_t)G::a_piece(wm * WM + j, g);
+  const uint32_t b_lane = lds_address(lds) + 2u * (uint32_t)(G::A_STAGE + G::b_chunk(8 * g + (j >> 2),
+                                                                                      wn * 64 + 4 * (j & 3)));
+  // Fragment read r (0..FM + 7) of k-half h of the stage at byte offset `at`
+  // of the ring: the k-half selects bit 6 of A's address, the column block bits
+  // 5 and 6 of B's (the swizzles are XORs).
+  short4_t b_lo;
+  auto read = [&](int h, uint32_t at, int r) {
+    if (r < 8) {
+      const int fn = r >> 1;
+      const uint32_t addr = ((b_lane + at) ^ (uint32_t)(32 * fn)) + (uint32_t)(64 * h) * G::SB;
+      if ((r & 1) == 0) {
+        b_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GG_LDS short4_t*)(uintptr_t)addr);
+      } else {
+        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GG_LDS short4_t*)(uintptr_t)(addr + 8u * G::SB));
+        b[h][fn] = __builtin_bit_cast(half8_t, __builtin_shufflevector(b_lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
     } else {
-      wait_vmcnt<PENDING>();
+      const int fm = r - 8;
+      a[h][fm] = *(const GG_LDS half8_t*)(uintptr_t)(((a_lane + at) ^ (uint32_t)(64 * h)) + (uint32_t)(32 * fm) * G::SA);
     }
-    if (stamped) stamps.step_mark(3);
-    if (k + 1 == loader.last_stage) loader.fix_last_stage(k + 1, lds + un * G::STAGE);
+  };
+  // The MFMAs of k-half h, among them the reads of the next half and
+  // issue(0 .. LOADS_N - 1).
+  auto phase = [&](int h, auto&& read_next, auto loads_tag, auto&& issue) {
+    constexpr int N = FM * 4;                         // MFMAs
+    constexpr int READS = FM + 8;
+    constexpr int LOADS_N = decltype(loads_tag)::value;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int fm = i >> 2, fn = (fm & 1) != 0 ? 3 - (i & 3) : i & 3;
+      acc[fm][fn] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[h][fn], a[h][fm], acc[fm][fn], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < READS; ++r) {
+        if (r * (N * 3 / 4) / READS == i) read_next(r);  // within the first three quarters
+      }
+#pragma unroll
+      for (int l = 0; l < LOADS_N; ++l) {
+        if (N - LOADS_N + l == i) issue(l);  // the last ones
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  const auto nothing = [](int) {};
+#pragma unroll
+  for (int r = 0; r < FM + 8; ++r) read(0, 0, r);
+
+  int t = 0, u = 0;  // stage and its buffer
+  // Stages with all the loads that follow still to be issued.
+#pragma unroll 1
+  for (; t < nk - NBUF; ++t) {
+    const int un = u == NBUF - 1 ? 0 : u + 1, ul = u == 0 ? NBUF - 1 : u - 1;
+    const uint32_t here = 2u * (uint32_t)(u * G::STAGE), next = 2u * (uint32_t)(un * G::STAGE);
+    const bool stamped = t == nk / 2;  // the step whose timing a traced launch records
+    if (stamped) stamps.step_mark(0);
+    const auto second = [&](int l) { loader.issue_load(t + NBUF - 1, lds + ul * G::STAGE, FIRST + l); };
+    phase(0, [&](int r) { read(1, here, r); }, std::integral_constant<int, LOADS - FIRST>{}, second);
+    if (stamped) stamps.step_mark(1);
+    if (t == 0 && extra) {
+      wait_vmcnt<(NBUF - 2) * LOADS + 1>();
+    } else {
+      wait_vmcnt<(NBUF - 2) * LOADS>();
+    }
+    if (stamped) stamps.step_mark(2);
     stage_barrier();
+    if (stamped) stamps.step_mark(3);
+    const auto first = [&](int l) { loader.issue_load(t + NBUF, lds + u * G::STAGE, l); };
+    phase(1, [&](int r) { read(0, next, r); }, std::integral_constant<int, FIRST>{}, first);
     if (stamped) stamps.step_mark(4);
     u = un;
   }
+  // The last stages: the rest of the last one's loads, then only waits.
+  const int tail = t;
+#pragma unroll 1
+  for (; t < nk; ++t) {
+    const int un = u == NBUF - 1 ? 0 : u + 1, ul = u == 0 ? NBUF - 1 : u - 1;
+    const uint32_t here = 2u * (uint32_t)(u * G::STAGE), next = 2u * (uint32_t)(un * G::STAGE);
+    const bool stamped = t == nk / 2;
+    if (stamped) stamps.step_mark(0);
+    if (FIRST < LOADS && t == tail && deep) {
+#pragma unroll
+      for (int l = FIRST; l < LOADS; ++l) loader.issue_load(t + NBUF - 1, lds + ul * G::STAGE, l);
+    }
+    phase(0, [&](int r) { read(1, here, r); }, std::integral_constant<int, 0>{}, nothing);
+    if (stamped) {
+      stamps.step_mark(1);
+      stamps.step_mark(2);
+    }
+    if (t + 1 < nk) {
+      // Loads of the stages after t + 1 may stay in flight, and the request made at the start.
+      const bool young = t == 0 && extra;
+      if (NBUF >= 4 && deep && t == tail) {
+        if (young) wait_vmcnt<2 * LOADS + 1>(); else wait_vmcnt<2 * LOADS>();
+      } else if (NBUF >= 3 && deep && t == tail + NBUF - 3) {
+        if (young) wait_vmcnt<LOADS + 1>(); else wait_vmcnt<LOADS>();
+      } else {
+        if (young) wait_vmcnt<1>(); else wait_vmcnt<0>();
+      }
+      if (t + 1 == loader.last_stage) loader.fix_last_stage(t + 1, lds + un * G::STAGE);
+      stage_barrier();
+    }
+    if (stamped) stamps.step_mark(3);
+    phase(1, [&](int r) { read(0, next, r); }, std::integral_constant<int, 0>{}, nothing);  // past K: unused
+    if (stamped) stamps.step_mark(4);
+    u = un;
+  }
+  // A traced launch's k-loop ends when every wave's does.
+  if constexpr (!std::is_same_v<Stamps, NoStamps>) phase_barrier();
 }
 
 // ---------------------------------------------------------------------------
@@ -245,7 +361,7 @@ struct MfmaTile {
     } else if constexpr (PHASED) {
       run_k_loop_phased<G>(p, m0, n0, lds, wm, wn, acc, on_start, stamps);
     } else {
-      run_k_loop_dma<G>(p, m0, n0, lds, compute, on_start, stamps);
+      run_k_loop_halves<G, WM>(p, m0, n0, lds, wm, wn, acc, on_start, stamps);
     }
     after_k_loop();
 

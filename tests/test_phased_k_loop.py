@@ -1,11 +1,13 @@
-"""The phased k-loop of the full 256 x 256 work tile (csrc/gg_phased.h) at the depths where it can go
-wrong: one, two and three stages (prologue, count-down stages and main loop), depths around the
-32-deep half stage and the 16-byte piece, odd depths and columns (2-byte aligned rows, repaired last
-pieces), partial tiles, and padding that holds infinities (nothing past K, M or N may reach D).
+"""The pipelined k-loops at the depths where they can go wrong: the phased one of the full 256 x 256
+work tile (csrc/gg_phased.h) and the one in halves of its edge classes (three and four stage buffers)
+and of the 128 x 128 work tile (two), csrc/gg_tiles.h.  One to six stages (fewer than the buffers,
+prologue, main loop and last stages), depths around the 32-deep half stage and the 16-byte piece, odd
+depths and columns (2-byte aligned rows, repaired last pieces), partial tiles, and padding that holds
+infinities (nothing past K, M or N may reach D).
 
-run_baseline_per_problem runs every tile with more than 128 rows and columns through it; the grouped
-launch of the same few problems runs on 128 x 128 work tiles with another k-loop and must give the
-same bits.  Against 64 bits: binary16 products are exact in binary32, so each of the K additions of an
+run_baseline_per_problem runs 256 x 256 work tiles (more than 128 rows and columns: the phased loop;
+else an edge class); the grouped launch of the same few problems runs on 128 x 128 work tiles and
+must give the same bits.  Against 64 bits: binary16 products are exact in binary32, so each of the K additions of an
 element rounds once, and alpha and beta C add two more roundings: |error| <= 2^-24 (K + 2)
 (|alpha| sum |a b| + |beta c|) (1 + 2^-20)."""
 import pytest
@@ -24,7 +26,8 @@ def test_depths_and_edges(torch_cuda, config, k):
     g = torch.Generator(device="cuda")
     g.manual_seed(1000 + k)
     probs, checks, keep = [], [], []
-    for m, n, pad in ((256, 256, 0), (129, 129, 0), (192, 255, 5), (300, 385, 3), (257, 131, 0)):
+    for m, n, pad in ((256, 256, 0), (129, 129, 0), (192, 255, 5), (300, 385, 3), (257, 131, 0), (100, 256, 0),
+                      (256, 100, 1), (37, 90, 0), (128, 128, 0), (1, 1, 0), (65, 129, 0)):
         lda, ldb, ldd = k + pad, n + pad, n + pad
         a = torch.full((m + 1, lda), float("inf"), device="cuda", dtype=torch.float16)
         b = torch.full((k + 1, ldb), float("inf"), device="cuda", dtype=torch.float16)
