@@ -191,12 +191,14 @@ SIGNATURES = {
     "ggk_work_halves_supported": (_i, [_i, _i]),
     "ggk_small_variant": (_i, [_i]),
     "ggk_launch_grouped": (_i, [_i, _i, _i, _vp, _vp, _vp, _vp, _i, _i, _vp, c_int_p, _i, _vp]),
+    "ggk_launch_grouped_done": (_i, [_i, _i, _i, _vp, _vp, _vp, _vp, _i, _i, _vp, c_int_p, _i, _vp, c_int_p, _vp]),
     "ggk_launch_grouped_traced": (_i, [_i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp, c_int_p, _i, _vp, _vp,
                                        _vp, _vp]),
     "ggk_launch_single": (_i, [_i, _i, _P(GGDeviceProblemDesc), _vp]),
     "ggk_moe_prepare": (_i, [_i, _i, _P(GGKMoeLayout), _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
     "ggk_moe_layout_check": (_i, [_i, _i, _P(GGKMoeLayout)]),
     "ggk_launch_grouped_device": (_i, [_i, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, _vp]),
+    "ggk_launch_grouped_device_done": (_i, [_i, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _i, _vp, c_int_p, _vp]),
     "ggk_kernel_resources_get": (_i, [_i, _i, _i, _P(GGKKernelResources)]),
     "ggk_occupancy": (_i, [_i, _i, c_int_p]),
     "ggk_fill_uniform_f16": (_i, [_vp, ctypes.c_int64, ctypes.c_uint64, ctypes.c_uint64, ctypes.c_float,

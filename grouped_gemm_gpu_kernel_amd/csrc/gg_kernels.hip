@@ -13,6 +13,7 @@
 //   gg_single_kernel   one problem, one workgroup per work tile
 //                      (single_problem_gemm_kernel, src/grouped_gemm.cu:677-688).
 //   fill kernels       synthetic inputs and output poisoning for tests/benches.
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -570,6 +571,28 @@ hipError_t ggk_event_create(hipEvent_t* event) {
 
 hipError_t ggk_event_destroy(hipEvent_t event) { return event == nullptr ? hipSuccess : hipEventDestroy(event); }
 
+// Launches a kernel and, when `done` is given, has its completion signal that
+// event (*recorded as for ggk_event_record_launch).  The signal belongs to the
+// kernel's own dispatch; recording the event after the launch puts a second
+// packet on the queue, which the next launch waits behind: back to back on one
+// stream a 2.3 us kernel takes 4.1 us with the first, 6.6 with the second.
+static hipError_t launch_kernel(const void* fn, dim3 grid, dim3 block, void** params, hipStream_t stream,
+                                hipEvent_t done, int* recorded) {
+  if (recorded != nullptr) *recorded = 0;
+  if (done != nullptr) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    hipError_t st = hipStreamIsCapturing(stream, &capture);
+    if (st != hipSuccess) return st;
+    if (capture == hipStreamCaptureStatusNone) {
+      st = hipExtLaunchKernel(fn, grid, block, params, 0, stream, nullptr, done, 0);
+      if (st == hipSuccess && recorded != nullptr) *recorded = GGK_LAUNCH_RECORDED;
+      return st;
+    }
+    if (recorded != nullptr) *recorded = GGK_LAUNCH_CAPTURED;
+  }
+  return hipLaunchKernel(fn, grid, block, params, 0, stream);
+}
+
 hipError_t ggk_event_record_launch(hipEvent_t event, hipStream_t stream, int* recorded) {
   if (recorded != nullptr) *recorded = 0;
   if (event == nullptr) return hipErrorInvalidValue;
@@ -639,7 +662,8 @@ static hipError_t launch_grouped(int variant, int path, int addressing, bool tra
                                  const int* d_work_offsets, const int* d_order, const int* d_work_table,
                                  int problem_count, int total_work, int* d_state, const int* chunk_bounds, int grid,
                                  int* d_tile_map, long long* d_wg_clock, long long* d_tile_phases,
-                                 hipStream_t stream) {
+                                 hipEvent_t done, int* recorded, hipStream_t stream) {
+  if (recorded != nullptr) *recorded = 0;
   if (!valid_kernel(variant, path) || grid <= 0 || problem_count < 0 || total_work < 0 ||
       (addressing != GGK_ADDR_32 && addressing != GGK_ADDR_64)) {
     return hipErrorInvalidValue;
@@ -656,8 +680,8 @@ static hipError_t launch_grouped(int variant, int path, int addressing, bool tra
   fill_bounds(args, chunk_bounds);
   void* params[] = {&args};
   const KernelSet& k = kKernels[variant][path];
-  return hipLaunchKernel(reinterpret_cast<const void*>(traced ? k.traced[addressing] : k.grouped[addressing]),
-                         dim3(grid), dim3(k.threads), params, 0, stream);
+  return launch_kernel(reinterpret_cast<const void*>(traced ? k.traced[addressing] : k.grouped[addressing]),
+                       dim3(grid), dim3(k.threads), params, stream, done, recorded);
 }
 
 // 32-bit offsets from a work tile's origin reach every A and B value the
@@ -710,13 +734,31 @@ hipError_t ggk_launch_grouped(int variant, int path, int addressing, const gg_de
                               const int* d_work_offsets, const int* d_order, const int* d_work_table,
                               int problem_count, int total_work, int* d_state, const int* chunk_bounds, int grid,
                               hipStream_t stream) {
+  return ggk_launch_grouped_done(variant, path, addressing, d_problems, d_work_offsets, d_order, d_work_table,
+                                 problem_count, total_work, d_state, chunk_bounds, grid, nullptr, nullptr, stream);
+}
+
+hipError_t ggk_launch_grouped_done(int variant, int path, int addressing, const gg_device_problem_desc* d_problems,
+                                   const int* d_work_offsets, const int* d_order, const int* d_work_table,
+                                   int problem_count, int total_work, int* d_state, const int* chunk_bounds, int grid,
+                                   hipEvent_t done, int* recorded, hipStream_t stream) {
   return launch_grouped(variant, path, addressing, false, d_problems, nullptr, d_work_offsets, d_order, d_work_table,
-                        problem_count, total_work, d_state, chunk_bounds, grid, nullptr, nullptr, nullptr, stream);
+                        problem_count, total_work, d_state, chunk_bounds, grid, nullptr, nullptr, nullptr, done,
+                        recorded, stream);
 }
 
 hipError_t ggk_launch_grouped_device(int variant, int path, int addressing, const gg_device_problem_desc* d_problems,
                                      const int* d_work_offsets, const int* d_order, int problem_count,
                                      const int* d_header, int* d_state, int grid, hipStream_t stream) {
+  return ggk_launch_grouped_device_done(variant, path, addressing, d_problems, d_work_offsets, d_order, problem_count,
+                                        d_header, d_state, grid, nullptr, nullptr, stream);
+}
+
+hipError_t ggk_launch_grouped_device_done(int variant, int path, int addressing,
+                                          const gg_device_problem_desc* d_problems, const int* d_work_offsets,
+                                          const int* d_order, int problem_count, const int* d_header, int* d_state,
+                                          int grid, hipEvent_t done, int* recorded, hipStream_t stream) {
+  if (recorded != nullptr) *recorded = 0;
   if (!valid_kernel(variant, path) || grid <= 0 || problem_count < 0 ||
       (addressing != GGK_ADDR_32 && addressing != GGK_ADDR_64)) {
     return hipErrorInvalidValue;
@@ -729,8 +771,8 @@ hipError_t ggk_launch_grouped_device(int variant, int path, int addressing, cons
                    nullptr, {}, d_header};
   void* params[] = {&args};
   const KernelSet& k = kKernels[variant][path];
-  return hipLaunchKernel(reinterpret_cast<const void*>(k.grouped[addressing]), dim3(grid), dim3(k.threads), params,
-                         0, stream);
+  return launch_kernel(reinterpret_cast<const void*>(k.grouped[addressing]), dim3(grid), dim3(k.threads), params,
+                       stream, done, recorded);
 }
 
 hipError_t ggk_launch_grouped_traced(int variant, int path, int addressing,
@@ -741,7 +783,7 @@ hipError_t ggk_launch_grouped_traced(int variant, int path, int addressing,
                                      hipStream_t stream) {
   return launch_grouped(variant, path, addressing, true, d_problems, d_tile_offsets, d_work_offsets, d_order,
                         d_work_table, problem_count, total_work, d_state, chunk_bounds, grid, d_tile_map, d_wg_clock,
-                        d_tile_phases, stream);
+                        d_tile_phases, nullptr, nullptr, stream);
 }
 
 hipError_t ggk_launch_single(int variant, int path, const gg_device_problem_desc* problem,

@@ -396,15 +396,11 @@ struct DeviceBuffer {
     return ggk_event_synchronize(last_launch);
   }
 
-  // Records the event after a launch on `stream`, or notes that the launch
-  // was captured.
-  hipError_t note_launch(hipStream_t stream) {
-    if (last_launch == nullptr) return hipSuccess;
-    int recorded = 0;
-    const hipError_t status = ggk_event_record_launch(last_launch, stream, &recorded);
+  // Notes a launch whose completion signals last_launch (GGK_LAUNCH_RECORDED)
+  // or that was captured (GGK_LAUNCH_CAPTURED).
+  void note_launch(int recorded) {
     if (recorded == GGK_LAUNCH_RECORDED) launched = true;
     if (recorded == GGK_LAUNCH_CAPTURED) captured = true;
-    return status;
   }
 
   // At least `bytes` on the current device, reusing the allocation when it is
@@ -927,13 +923,14 @@ hipError_t GroupedGemmExecutor::run(hipStream_t stream) const {
   if (impl_ == nullptr) return hipErrorInvalidDevicePointer;
   if (impl_->failed) return hipErrorInvalidValue;
   if (impl_->total_tiles == 0 || impl_->problem_count == 0) return hipSuccess;
-  const hipError_t status =
-      ggk_launch_grouped(impl_->variant, impl_->path, impl_->addressing, impl_->d_problems,
-                         impl_->d_ints + impl_->problem_count + 1, impl_->d_ints + 2 * (impl_->problem_count + 1),
-                         impl_->d_work_table(), impl_->problem_count, impl_->launch_total, impl_->d_state,
-                         impl_->launch_bounds.data(), impl_->grid_ctas, stream);
-  if (status != hipSuccess) return status;
-  return impl_->buffer.note_launch(stream);
+  int recorded = 0;
+  const hipError_t status = ggk_launch_grouped_done(
+      impl_->variant, impl_->path, impl_->addressing, impl_->d_problems, impl_->d_ints + impl_->problem_count + 1,
+      impl_->d_ints + 2 * (impl_->problem_count + 1), impl_->d_work_table(), impl_->problem_count,
+      impl_->launch_total, impl_->d_state, impl_->launch_bounds.data(), impl_->grid_ctas,
+      impl_->buffer.last_launch, &recorded, stream);
+  if (status == hipSuccess) impl_->buffer.note_launch(recorded);
+  return status;
 }
 
 hipError_t GroupedGemmExecutor::run_traced(int* d_tile_map, long long* d_wg_clock, hipStream_t stream,
@@ -941,13 +938,16 @@ hipError_t GroupedGemmExecutor::run_traced(int* d_tile_map, long long* d_wg_cloc
   if (impl_ == nullptr) return hipErrorInvalidDevicePointer;
   if (impl_->failed) return hipErrorInvalidValue;
   if (impl_->total_tiles == 0 || impl_->problem_count == 0) return hipSuccess;
-  const hipError_t status = ggk_launch_grouped_traced(
+  hipError_t status = ggk_launch_grouped_traced(
       impl_->variant, impl_->path, impl_->addressing, impl_->d_problems, impl_->d_ints,
       impl_->d_ints + impl_->problem_count + 1, impl_->d_ints + 2 * (impl_->problem_count + 1), impl_->d_work_table(),
       impl_->problem_count, impl_->launch_total, impl_->d_state, impl_->launch_bounds.data(), impl_->grid_ctas, d_tile_map,
       d_wg_clock, d_tile_phases, stream);
-  if (status != hipSuccess) return status;
-  return impl_->buffer.note_launch(stream);
+  if (status != hipSuccess || impl_->buffer.last_launch == nullptr) return status;
+  int recorded = 0;
+  status = ggk_event_record_launch(impl_->buffer.last_launch, stream, &recorded);
+  impl_->buffer.note_launch(recorded);
+  return status;
 }
 
 int GroupedGemmExecutor::problem_count() const { return impl_ != nullptr ? impl_->problem_count : 0; }
@@ -1292,12 +1292,13 @@ hipError_t MoeGroupedGemm::run(const int* d_counts, hipStream_t stream) const {
                                       impl_->d_problems, impl_->offsets(), impl_->perm(), impl_->order(),
                                       impl_->header(), stream);
   if (status != hipSuccess) return status;
-  status = ggk_launch_grouped_device(impl_->variant, impl_->path, impl_->addressing, impl_->d_problems,
-                                     impl_->offsets() + impl_->layout.experts + 1, impl_->order(),
-                                     impl_->layout.experts, impl_->header(), impl_->d_state, impl_->grid_ctas,
-                                     stream);
-  if (status != hipSuccess) return status;
-  return impl_->buffer.note_launch(stream);
+  int recorded = 0;
+  status = ggk_launch_grouped_device_done(impl_->variant, impl_->path, impl_->addressing, impl_->d_problems,
+                                          impl_->offsets() + impl_->layout.experts + 1, impl_->order(),
+                                          impl_->layout.experts, impl_->header(), impl_->d_state, impl_->grid_ctas,
+                                          impl_->buffer.last_launch, &recorded, stream);
+  if (status == hipSuccess) impl_->buffer.note_launch(recorded);
+  return status;
 }
 
 int MoeGroupedGemm::grid_ctas() const { return impl_ != nullptr ? impl_->grid_ctas : 0; }
