@@ -77,7 +77,7 @@ struct GroupedArgs {
 // the tiles of one problem, which share A and B panels, are then multiplied
 // on one XCD and its L2 serves the re-reads.  Workgroup w's first tile is
 // fixed, index bounds[home] + w / kChunks, so a launch starts without any
-// counter traffic; the rest of chunk c, [bounds[c] + fixed_slots(c),
+// counter traffic and without waiting for LDS; the rest of chunk c, [bounds[c] + fixed_slots(c),
 // bounds[c + 1]), is handed out one index per atomicAdd on the chunk's
 // counter.  A counter request takes microseconds (device-scope atomics are
 // resolved past the XCDs' L2s), so it is made while the current tile is being
@@ -96,22 +96,27 @@ __device__ __forceinline__ int counted_from(const int* bounds, int c, int grid) 
   return bounds[c] + fixed_slots(c, grid);
 }
 
-// The first visit at or after `visit` whose chunk has indices for its counter
-// to hand out (kChunks if none).
-__device__ __forceinline__ int first_counted(const int* bounds, int grid, int home, int visit) {
-  for (; visit < kChunks; ++visit) {
-    const int c = (home + visit) & (kChunks - 1);
-    if (counted_from(bounds, c, grid) < bounds[c + 1]) break;
-  }
-  return visit;
+// Bit c: chunk c has indices for its counter to hand out (wave 0).
+__device__ __forceinline__ uint32_t counted_chunks(const int* bounds, int grid) {
+  const int lane = threadIdx.x & (kWave - 1);
+  return (uint32_t)__ballot(lane < kChunks && counted_from(bounds, lane & (kChunks - 1), grid) <
+                                                  bounds[(lane & (kChunks - 1)) + 1]);
+}
+
+// The first visit at or after `visit` whose chunk is in the set `chunks`
+// (kChunks if none).
+__device__ __forceinline__ int first_counted(uint32_t chunks, int home, int visit) {
+  const uint32_t from_home = ((chunks >> home) | (chunks << (kChunks - home))) & ((1u << kChunks) - 1);
+  const uint32_t left = visit < kChunks ? from_home >> visit : 0u;
+  return left != 0 ? visit + __builtin_ctz(left) : kChunks;
 }
 
 // Claims an index now (wave 0): one lane per remaining chunk reads that
 // chunk's counter, the first chunk with indices left is asked, and the search
 // goes on past it if the request comes back empty.  Counters only grow
-// during a launch, so a chunk read as dry stays dry.  Returns total, with
+// during a launch, so a chunk read as dry stays dry.  Returns -1, with
 // visit = kChunks, when every chunk is exhausted.
-__device__ __forceinline__ int claim_now(int* state, const int* bounds, int grid, int home, int& visit, int total) {
+__device__ __forceinline__ int claim_now(int* state, const int* bounds, int grid, int home, int& visit) {
   const int lane = threadIdx.x & (kWave - 1);
   while (visit < kChunks) {
     bool open = false;
@@ -135,23 +140,31 @@ __device__ __forceinline__ int claim_now(int* state, const int* bounds, int grid
     ++visit;
   }
   visit = kChunks;
-  return total;
+  return -1;
 }
 
-// The schedule of one launch in LDS: s[0, kChunks] the chunk bounds, s[kChunks + 1]
-// the work-tile total, from the arguments or from the device header.
-__device__ __forceinline__ void load_schedule(const GroupedArgs& args, int* s) {
+// The chunk bounds of one launch in LDS, s[0, kChunks], from the arguments or
+// from the device header: written and read by wave 0 only, so no barrier.
+__device__ __forceinline__ void load_schedule(const GroupedArgs& args, int split, int* s) {
   const int tid = threadIdx.x;
   if (args.header != nullptr) {
-    if (tid <= kChunks) s[tid] = args.header[2 + tid];
-    if (tid == kChunks + 1) s[tid] = args.header[1];
+    if (tid <= kChunks) s[tid] = args.header[2 + tid] << split;
   } else {
 #pragma unroll
     for (int c = 0; c <= kChunks; ++c) {
       if (tid == c) s[c] = args.bounds[c];
     }
-    if (tid == kChunks + 1) s[tid] = args.total;
   }
+}
+
+// Bound c (wave-uniform) of the chunks, by scalar loads: the first tile is
+// found without waiting for LDS.
+__device__ __forceinline__ int chunk_bound(const GroupedArgs& args, int split, int c) {
+  if (args.header != nullptr) return ((const_int_ptr)args.header)[2 + c] << split;
+  int b = args.bounds[0];
+#pragma unroll
+  for (int i = 1; i <= kChunks; ++i) b = c == i ? args.bounds[i] : b;
+  return b;
 }
 
 // Index of the problem that owns index t: the number of problems p with
@@ -239,7 +252,7 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
   using G = typename S::G;
   __shared__ __attribute__((aligned(16))) uint16_t lds[KernelLds<S>::HALVES];
   __shared__ int s_claim[2];
-  __shared__ int s_schedule[kChunks + 2];
+  __shared__ int s_schedule[kChunks + 1];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -253,21 +266,32 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
 
   const int grid = gridDim.x;
   const int home = blockIdx.x % kChunks;
-  load_schedule(args, s_schedule);
-  __syncthreads();
-  const int total = __builtin_amdgcn_readfirstlane(s_schedule[kChunks + 1]);
-  // Whether any chunk has indices beyond the fixed first tiles: when none has,
-  // no counter is touched and none needs resetting.
-  const bool counted = first_counted(s_schedule, grid, 0, 0) < kChunks;
+  // A device-prepared launch of at most half as many work tiles as workgroups
+  // (the host does not know how many there are) claims each tile as its two
+  // column halves, indices 2 i and 2 i + 1: the other half of the chip would
+  // have nothing to do.  16 experts, 512 tokens, K 1024, N 2048 (120 tiles):
+  // 26.5 -> 21.0 us.  Above half, some workgroups would get two halves, which
+  // cost more than the one tile.
+  constexpr bool kSplits = S::CLASSES && !TRACED && !WIDE;
+  const int split =
+      kSplits && args.header != nullptr && 2 * ((const_int_ptr)args.header)[1] <= grid ? 1 : 0;
+  int t = chunk_bound(args, split, home) + (int)blockIdx.x / kChunks;
+  const bool fixed = t < chunk_bound(args, split, home + 1);
+  // Wave 0: the chunks with indices beyond the fixed first tiles.  When there
+  // is none, no counter is touched and none needs resetting.
+  uint32_t counted = 0;
+  if (wave0) {
+    load_schedule(args, split, s_schedule);
+    counted = counted_chunks(s_schedule, grid);
+  }
 
   int visit = 0;  // wave 0
-  int t = __builtin_amdgcn_readfirstlane(s_schedule[home] + (int)blockIdx.x / kChunks);
   int parity = 0;
-  if (t >= __builtin_amdgcn_readfirstlane(s_schedule[home + 1])) {
+  if (!fixed) {
     // No fixed tile for this workgroup (its chunk is smaller than its share
     // of the grid): claim one now.
     if (wave0) {
-      const int c = counted ? claim_now(args.state, s_schedule, grid, home, visit, total) : total;
+      const int c = counted != 0 ? claim_now(args.state, s_schedule, grid, home, visit) : -1;
       if (lane == 0) s_claim[0] = c;
     }
     __syncthreads();
@@ -275,15 +299,15 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
     parity = 1;
   }
 
-  while (t < total) {
+  while (t >= 0) {
     // The request for the next index, made once while this tile is computed.
     bool asked = false;
     int chunk = -1;  // wave 0: the chunk asked, -1 if none
     int got = 0;     // wave 0, lane 0: what the request returned
     auto request = [&]() -> bool {
       asked = true;
-      if (!wave0 || !counted) return false;
-      visit = first_counted(s_schedule, grid, home, visit);
+      if (!wave0) return false;
+      visit = first_counted(counted, home, visit);
       if (visit >= kChunks) return false;
       chunk = (home + visit) & (kChunks - 1);
       if (lane == 0) got = atomicAdd(args.state + chunk * kStride, 1);
@@ -299,16 +323,16 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
     // store (the epilogue reads no LDS, and the barrier after the k-loop has
     // seen every LDS read of this tile).  Slot `parity` was last read before
     // the previous tile's handover barrier.
-    int next_t = total;
+    int next_t = -1;
     bool handed = false;
     auto hand_over = [&]() {
       if (wave0) {
-        int next = total;
+        int next = -1;
         if (chunk >= 0) {
           next = counted_from(s_schedule, chunk, grid) + __builtin_amdgcn_readfirstlane(got);
           if (next >= s_schedule[chunk + 1]) {
             ++visit;
-            next = claim_now(args.state, s_schedule, grid, home, visit, total);
+            next = claim_now(args.state, s_schedule, grid, home, visit);
           }
         }
         if (lane == 0) s_claim[parity] = next;
@@ -338,9 +362,10 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
       local = word & GGK_WORK_LOCAL_MASK;
       half = S::CLASSES ? (word >> GGK_WORK_HALF_SHIFT) & 3 : 0;
     } else {
-      const int pos = find_problem(args.work_offsets, args.count, t);
+      const int tile = t >> split;
+      const int pos = find_problem(args.work_offsets, args.count, tile);
       prob = args.order != nullptr ? ((const_int_ptr)args.order)[pos] : pos;
-      local = t - ((const_int_ptr)args.work_offsets)[pos];
+      local = tile - ((const_int_ptr)args.work_offsets)[pos];
     }
     // Uniform index into read-only memory: scalar loads of the 80-byte descriptor.
     const gg_device_problem_desc p = load_problem(args.problems, prob);
@@ -366,18 +391,20 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
           }
         }
       } else {
-        // One half of the rows (whole rows of macro-tiles) is computed as a
-        // problem that ends with that half: its tile has at most BM / 2 rows
-        // and runs in a half-height edge class, and each of its D elements is
-        // computed as in the whole tile.
+        // One half of the rows (whole rows of macro-tiles) or of the columns is
+        // computed as a problem that ends with that half: its tile has at most
+        // BM / 2 rows (BN / 2 columns) and runs in an edge class, and each of its
+        // D elements is computed as in the whole tile.
         gg_device_problem_desc q = p;
         const int m0 = wm * G::BM + (half == 2 ? G::BM / 2 : 0);
         if (half != 0 && m0 + G::BM / 2 < p.m) q.m = m0 + G::BM / 2;
+        const int n0 = wn * G::BN + (split != 0 && (t & 1) != 0 ? G::BN / 2 : 0);
+        if (split != 0 && n0 + G::BN / 2 < p.n) q.n = n0 + G::BN / 2;
         if constexpr (TRACED) {
-          mark_tile_start<G>(stamps, half, q, m0, wn * G::BN);
-          run_work_tile<S, PATH, WIDE>(q, m0, wn * G::BN, lds, request, after_k_loop, stamps);
-        } else {
-          run_work_tile<S, PATH, WIDE>(q, m0, wn * G::BN, lds, request, after_k_loop);
+          mark_tile_start<G>(stamps, half, q, m0, n0);
+          run_work_tile<S, PATH, WIDE>(q, m0, n0, lds, request, after_k_loop, stamps);
+        } else if (!kSplits || n0 < p.n) {  // else: an empty second half
+          run_work_tile<S, PATH, WIDE>(q, m0, n0, lds, request, after_k_loop);
         }
       }
     }
@@ -397,7 +424,7 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
     // request in flight, so when the last one leaves nobody will touch the
     // counters again: it returns them to zero for the next launch in stream
     // order.
-    if (counted) {
+    if (counted != 0) {
       const int retired = atomicAdd(args.state + kChunks * kStride, 1);
       if (retired == grid - 1) {
         for (int c = 0; c <= kChunks; ++c) atomicExch(args.state + c * kStride, 0);
