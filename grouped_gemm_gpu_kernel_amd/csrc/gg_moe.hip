@@ -81,6 +81,31 @@ __device__ __forceinline__ void least_from(unsigned long long& v, int& idx) {
   idx = take ? pidx : idx;
 }
 
+// Number of the wave's first `count` lanes whose (key, lane) precedes this
+// lane's: larger keys first, ties to the lower lane.  Keys pass through scalar
+// registers, so a step is a handful of independent compares; counting over LDS
+// (as larger groups do) waits for its reads.
+__device__ __forceinline__ int wave_rank(unsigned long long key, int count) {
+  const int lane = threadIdx.x % kWave;
+  const int lo = (int)(uint32_t)key, hi = (int)(uint32_t)(key >> 32);
+  int rank = 0;
+#pragma unroll 4
+  for (int j = 0; j < count; ++j) {
+    const unsigned long long other = ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane(hi, j) << 32) |
+                                     (uint32_t)__builtin_amdgcn_readlane(lo, j);
+    rank += (other > key || (other == key && j < lane)) ? 1 : 0;
+  }
+  return rank;
+}
+
+// The lesser of this lane's value and lane i + SH's (as least_from).
+template <int SH>
+__device__ __forceinline__ double least_of(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x100 + SH, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x100 + SH, 0xf, 0xf, false);
+  return __builtin_fmin(v, __hiloint2double(hi, lo));
+}
+
 // Exclusive prefix sum of one value per thread over the workgroup of THREADS
 // threads, in thread order; *total receives the sum.  Every thread must call it.
 template <int THREADS, class T>
@@ -175,7 +200,14 @@ __global__ __launch_bounds__(THREADS) void moe_prepare_kernel(MoeArgs args) {
   // by K, larger k first, then larger m * n; by tiles, more tiles first, then
   // the by-K order.  Every expert has the same k here, so ties fall to m * n,
   // then to the expert index.
-  if (tid < experts) {
+  if constexpr (THREADS == kWave) {
+    // Every expert has the same n, so m * n orders as the rows do.
+    const bool in = tid < experts, by_tiles = args.sort_mode == 2 || args.sort_mode == 3;
+    const uint32_t k1 = in && by_tiles ? (uint32_t)s_tiles[tid] : 0u;
+    const uint32_t k0 = in && L.n > 0 ? (uint32_t)s_rows[tid] : 0u;
+    const int rank = args.sort_mode != 0 ? wave_rank(((unsigned long long)k1 << 32) | k0, experts) : tid;
+    if (in) s_perm[rank] = tid;
+  } else if (tid < experts) {
     int rank = tid;
     if (args.sort_mode != 0) {
       const bool tiles_first = args.sort_mode == 2 || args.sort_mode == 3;
@@ -271,7 +303,13 @@ __global__ __launch_bounds__(THREADS) void moe_prepare_kernel(MoeArgs args) {
   long long sum_all;
   (void)block_exclusive_scan<THREADS, long long>(total, s_waves_ll, &sum_all);
   const long long share = sum_all / kChunks + (sum_all % kChunks != 0 ? 1 : 0);
-  if (pos < experts) {
+  if constexpr (THREADS == kWave) {
+    const int rank = wave_rank((unsigned long long)total, experts);
+    if (pos < experts) {
+      s_by_total[rank] = total;
+      s_order[rank] = pos;
+    }
+  } else if (pos < experts) {
     int rank = 0;
 #pragma unroll 8
     for (int j = 0; j < experts; ++j) {
@@ -290,7 +328,38 @@ __global__ __launch_bounds__(THREADS) void moe_prepare_kernel(MoeArgs args) {
   // each step takes its own from its lane and leaves its choice in that lane.
   // Returns each lane's final load.
   const int lane = tid & (kWave - 1);
+  // While eight times every load stays below 2^53 (anything but absurd sizes),
+  // a chunk's load and number are one exact double, 8 load + number: the least
+  // is then three 64-bit minima, and the lane it belongs to is the one that
+  // holds it (340 cycles a position for the pairs below, 64 experts).
+  const bool exact = sum_all < (1LL << 50);
   auto greedy = [&](int from, unsigned long long load) {
+    if (exact) {
+      const bool closed = load == ~0ull;
+      double mine_key = closed ? __builtin_huge_val() : (double)(8 * load + (unsigned long long)lane);
+      for (int r0 = from; r0 < experts; r0 += kWave) {
+        const int r = r0 + lane;
+        const double step = r < experts ? (double)(8 * s_by_total[r]) : 0.0;
+        const int lo = __double2loint(step), hi = __double2hiint(step);
+        const int steps = min(kWave, experts - r0);
+        int chosen = 0;
+        for (int j = 0; j < steps; ++j) {
+          const double t = __hiloint2double(__builtin_amdgcn_readlane(hi, j), __builtin_amdgcn_readlane(lo, j));
+          double v = mine_key;
+          v = least_of<4>(v);
+          v = least_of<2>(v);
+          v = least_of<1>(v);
+          const double least = __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                                                __builtin_amdgcn_readfirstlane(__double2loint(v)));
+          const bool owner = mine_key == least;
+          const int best = __builtin_ctzll(__ballot(owner));
+          mine_key = owner ? mine_key + t : mine_key;
+          chosen = lane == j ? best : chosen;
+        }
+        if (r < experts) s_chunk[s_order[r]] = chosen;
+      }
+      return closed ? load : (unsigned long long)mine_key >> 3;
+    }
     for (int r0 = from; r0 < experts; r0 += kWave) {
       const int r = r0 + lane;
       const unsigned long long mine = r < experts ? (unsigned long long)s_by_total[r] : 0ull;
@@ -363,7 +432,21 @@ __global__ __launch_bounds__(THREADS) void moe_prepare_kernel(MoeArgs args) {
   }
   __syncthreads();
   int chunk = 0;
-  if (pos < experts) {
+  if constexpr (THREADS == kWave) {
+    chunk = pos < experts ? s_chunk[pos] : 0;
+    const int key_lo = __double2loint(key), key_hi = __double2hiint(key);
+    int before = 0;  // positions scheduled ahead of this one
+#pragma unroll 4
+    for (int j = 0; j < experts; ++j) {
+      const int cj = __builtin_amdgcn_readlane(chunk, j);
+      const double kj = __hiloint2double(__builtin_amdgcn_readlane(key_hi, j), __builtin_amdgcn_readlane(key_lo, j));
+      before += (cj < chunk || (cj == chunk && (kj > key || (kj == key && j < pos)))) ? 1 : 0;
+    }
+    if (pos < experts) {
+      if (chunk >= 0) atomicAdd(&s_chunk_work[chunk], work);
+      s_order[before] = pos;  // its by-total contents were last read by the greedy pass
+    }
+  } else if (pos < experts) {
     chunk = s_chunk[pos];
     int before = 0;  // positions scheduled ahead of this one
 #pragma unroll 2
