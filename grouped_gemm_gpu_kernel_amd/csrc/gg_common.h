@@ -47,7 +47,7 @@ constexpr int kWave = 64;
 // loads of stage k + DEPTH - 1 issued while stage k is multiplied (a ring of
 // DEPTH register sets), written to two LDS buffers.  Loads straight into LDS
 // use BUFFERS LDS buffers, BUFFERS - 1 stages in flight.
-template <int BM_, int BN_, int BK_, int DEPTH_, int THREADS_, int BUFFERS_ = 2, bool A_SWIZZLED_ = false>
+template <int BM_, int BN_, int BK_, int DEPTH_, int THREADS_, int BUFFERS_ = 2>
 struct Geometry {
   static constexpr int BM = BM_;
   static constexpr int BN = BN_;
@@ -55,14 +55,10 @@ struct Geometry {
   static constexpr int DEPTH = DEPTH_;
   static constexpr int THREADS = THREADS_;
   static constexpr int BUFFERS = BUFFERS_;
-  // Swizzled, unpadded A rows (needed by loads straight into LDS), or rows
-  // padded by 8 values (the FMA tile, whose operand reads then need no
-  // per-piece index arithmetic).
-  static constexpr bool A_SWIZZLED = A_SWIZZLED_;
   static_assert(DEPTH >= 2, "at least one stage must be in flight while another is multiplied");
   static_assert(BUFFERS >= 2, "at least double buffered");
   static_assert(THREADS % kWave == 0, "whole waves");
-  static constexpr int SA = A_SWIZZLED ? BK : BK + 8;
+  static constexpr int SA = BK;  // unpadded: loads straight into LDS write whole rows
   static constexpr int SB = BN;
   static constexpr int APR = BK / 8;  // 16-byte pieces per A row
   static_assert(APR == 4 || APR == 8, "A swizzle is defined for 32- and 64-deep stages");
@@ -99,7 +95,7 @@ struct Geometry {
   // A: rows that share a 256-byte bank window (row / RPW equal) get distinct
   // piece positions; RPW = 256 / (2 BK) rows per window.
   static constexpr int A_RPW = 128 / BK;
-  __device__ static __forceinline__ int a_swizzle(int row) { return A_SWIZZLED ? (row / A_RPW) & (APR - 1) : 0; }
+  __device__ static __forceinline__ int a_swizzle(int row) { return (row / A_RPW) & (APR - 1); }
   // Element offset, within an A stage, of the 16-byte piece c (values 8c ..
   // 8c + 7 of the stage's k range) of a row.
   __device__ static __forceinline__ int a_piece(int row, int c) { return row * SA + 8 * (c ^ a_swizzle(row)); }
@@ -107,9 +103,6 @@ struct Geometry {
 
 #ifndef GG_STAGE_K
 #define GG_STAGE_K 64
-#endif
-#ifndef GG_STAGE_DEPTH
-#define GG_STAGE_DEPTH 3
 #endif
 
 // Reference macro-tile of each variant (ids follow GGK_VARIANT_*).
@@ -184,7 +177,7 @@ template <int V> struct KernelShape<V, GGK_PATH_MFMA> {
   // two stages keeps it within the registers beside the accumulators (the
   // 256 x 256 work tile's still spills: launches route that form to the
   // 128 x 128 work tile of the same macro-tile).
-  using G = Geometry<BM, BN, GG_STAGE_K, 2, THREADS, BUFFERS, true>;
+  using G = Geometry<BM, BN, GG_STAGE_K, 2, THREADS, BUFFERS>;
   // Edge classes of the 256 x 256 work tile (32-bit addressing form): a work
   // tile with at most BM / 2 rows or BN / 2 columns inside the problem stages
   // only that half of A or B, so a stage is 48 KB (32 KB when both) and three
@@ -194,16 +187,19 @@ template <int V> struct KernelShape<V, GGK_PATH_MFMA> {
   // element is still one lane's 16x16x32 MFMA chain over ascending k with the
   // same epilogue, so D does not depend on the class.
   static constexpr bool CLASSES = GG_TILE_CLASSES != 0 && kLarge && BM == 256 && BN == 256 && THREADS == 512;
-  using GR = Geometry<BM / 2, BN, GG_STAGE_K, 2, THREADS, 3, true>;       // rows <= BM / 2
-  using GC = Geometry<BM, BN / 2, GG_STAGE_K, 2, THREADS, 3, true>;       // columns <= BN / 2
-  using GRC = Geometry<BM / 2, BN / 2, GG_STAGE_K, 2, THREADS, 4, true>;  // both
+  using GR = Geometry<BM / 2, BN, GG_STAGE_K, 2, THREADS, 3>;       // rows <= BM / 2
+  using GC = Geometry<BM, BN / 2, GG_STAGE_K, 2, THREADS, 3>;       // columns <= BN / 2
+  using GRC = Geometry<BM / 2, BN / 2, GG_STAGE_K, 2, THREADS, 4>;  // both
   static constexpr int WAVE_M_R = 64, WAVE_M_C = 64, WAVE_M_RC = 32;
 };
 template <int V> struct KernelShape<V, GGK_PATH_FMA> {
   static constexpr int TM = 1;
   static constexpr int TN = 1;
-  static constexpr int WAVES_PER_EU = 2;
-  using G = Geometry<VariantTile<V>::M, VariantTile<V>::N, GG_STAGE_K, GG_STAGE_DEPTH, 256>;
+  // A 64 x 64 tile needs 128 registers and 32 KB of LDS: four workgroups a CU.
+  // The larger tiles need more than a third of the registers (at three waves
+  // per SIMD they spill).
+  static constexpr int WAVES_PER_EU = VariantTile<V>::M * VariantTile<V>::N <= 64 * 64 ? 4 : 2;
+  using G = Geometry<VariantTile<V>::M, VariantTile<V>::N, GG_STAGE_K, 2, 256>;
   static constexpr bool CLASSES = false;
 };
 
@@ -329,15 +325,8 @@ __device__ __forceinline__ u32x4_t finish_piece(const RawPiece& r, uint32_t lead
 }
 
 // The loads of one stage in flight: this thread's A and B pieces.
-template <class G, bool WIDE>
-struct RawStage;
 template <class G>
-struct RawStage<G, false> {
-  u32x4_t a[G::A_PER_THREAD];
-  u32x4_t b[G::B_PER_THREAD];
-};
-template <class G>
-struct RawStage<G, true> {
+struct RawStage {
   RawPiece a[G::A_PER_THREAD];
   RawPiece b[G::B_PER_THREAD];
 };
@@ -350,10 +339,6 @@ struct RawStage<G, true> {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, int64_t bytes) {
   const int64_t n = bytes < 0 ? 0 : (bytes > 0xffffffffll ? 0xffffffffll : bytes);
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)(uint32_t)n, 0x00020000);
-}
-
-__device__ __forceinline__ u32x4_t buffer_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
 }
 
 // Replaces binary16 value idx of a 16-byte piece with h (low 16 bits); an idx
@@ -385,7 +370,9 @@ __device__ __forceinline__ u32x4_t keep_values(u32x4_t v, int n) {
   return v;
 }
 
-// Moves the A and B stages of one work tile from global memory into LDS.
+// Moves the A and B stages of one work tile from global memory into LDS
+// through registers, with 64-bit addresses (DmaLoader serves tiles whose
+// offsets fit in 32 bits; the host picks the form, see fits_addr32).
 //
 // A piece v (v = tid + THREADS * i) covers tile row v / (BK/8), columns
 // 8 * (v % (BK/8)) of the stage; B piece v covers k-row v / (BN/8), columns
@@ -396,126 +383,17 @@ __device__ __forceinline__ u32x4_t keep_values(u32x4_t v, int n) {
 // that are never stored and may hold anything.  Values at k >= K meet each
 // other in the products, so both operands are zeroed there.
 //
-// WIDE = false: every piece is one 16-byte buffer load at its exact byte
-// offset (2-byte aligned rows need no realignment), through a buffer resource
-// that spans from the tile's origin to the end of the matrix: rows of A past
-// M and rows of B past K lie beyond it (for ld >= the row length) and read as
-// zero without touching memory, and nothing past the matrix is ever read.  A
-// values at k >= K (the next row's head) and B rows at k >= K are zeroed when
-// the stage is written.  Every stage issues the same loads, with no branch,
-// so the compiler can count the loads in flight exactly.  The host selects
-// this form when the per-tile byte offsets fit in 31 bits
-// (rows * lda < 2^30, stage_k * ldb < 2^30, non-negative ld).  The range check
-// works on the access's dwords: when a piece starts 2 bytes past a dword, the
-// dword that holds the matrix's last value reaches 2 bytes past the matrix
-// and reads as 0, so the last value of A and of B is read separately (through
-// its aligned dword) and put back when the last stage is written.
-//
-// WIDE = true: 64-bit addresses per piece; each piece is fetched as the
-// dwords from the 4-byte aligned address at or below it that hold wanted
-// values (a dword past them is fetched from the first one again) and shifted
-// into place when written; values outside the matrix are zero-filled.
-template <class G, bool WIDE>
-struct StageLoader;
-
+// Each piece is fetched as the dwords from the 4-byte aligned address at or
+// below it that hold wanted values (a dword past them is fetched from the
+// first one again) and shifted into place when written; values outside the
+// matrix are zero-filled.
 template <class G>
-struct StageLoader<G, false> {
+struct StageLoader {
   static constexpr int T = G::THREADS;
   static constexpr int NA = G::A_PER_THREAD;
   static constexpr int NB = G::B_PER_THREAD;
   static constexpr int APR = G::BK / 8;  // A pieces per row
   static constexpr int BPR = G::BN / 8;  // B pieces per k-row
-  // LDS distance between a thread's consecutive pieces.  The B swizzle
-  // repeats every 16 k-rows, so it is the same for all of a thread's pieces.
-  static constexpr int A_LDS_STEP = (T / APR) * G::SA;
-  static constexpr int B_LDS_STEP = (T / BPR) * G::SB;
-  static_assert((T / BPR) % 16 == 0, "a thread's B pieces must share their swizzle");
-  static_assert(!G::A_SWIZZLED || (T / APR) % (G::A_RPW * APR) == 0, "a thread's A pieces must share their swizzle");
-
-  const gg_device_problem_desc& p;
-  __amdgpu_buffer_rsrc_t a_rsrc;  // A from (m0, 0) to the matrix end
-  const uint16_t* b_tile;         // B at (0, n0)
-  int64_t b_bytes;                // bytes from b_tile to the end of B
-  uint32_t a_off, b_off;          // byte offset of this thread's piece 0 from its origin
-  uint32_t a_step, b_step;        // byte distance between a thread's pieces (wave-uniform)
-  int a_lds, b_lds;               // LDS offset (values) of piece 0 within a stage's A / B part
-  int m0, n0;
-  int last_stage;                 // index of the stage that holds k = K - 1
-  uint32_t a_last, b_last;        // A[m-1][k-1] and B[k-1][n-1]
-
-  __device__ __forceinline__ StageLoader(const gg_device_problem_desc& prob, int m0_, int n0_)
-      : p(prob), m0(m0_), n0(n0_) {
-    const int tid = opaque_tid();
-    const uint16_t* A = static_cast<const uint16_t*>(p.a);
-    const uint16_t* B = static_cast<const uint16_t*>(p.b);
-    const uint16_t* a_tile = A + (int64_t)m0 * p.lda;
-    // Last element of A is (m - 1, k - 1); of B, (k - 1, n - 1).
-    a_rsrc = buffer_rsrc(a_tile, 2 * ((int64_t)(p.m - 1 - m0) * p.lda + p.k));
-    b_tile = B + n0;
-    b_bytes = 2 * ((int64_t)(p.k - 1) * p.ldb + p.n - n0);
-    a_off = 2u * ((uint32_t)(tid / APR) * (uint32_t)p.lda + (uint32_t)(8 * (tid % APR)));
-    b_off = 2u * ((uint32_t)(tid / BPR) * (uint32_t)p.ldb + (uint32_t)(8 * (tid % BPR)));
-    a_step = 2u * (uint32_t)(T / APR) * (uint32_t)p.lda;
-    b_step = 2u * (uint32_t)(T / BPR) * (uint32_t)p.ldb;
-    a_lds = G::a_piece(tid / APR, tid % APR);  // the thread's pieces share the swizzle (rows 64 apart)
-    b_lds = G::b_chunk(tid / BPR, 8 * (tid % BPR));
-    last_stage = (p.k - 1) / G::BK;
-    a_last = p.k > 0 ? load_value_uniform(A + (int64_t)(p.m - 1) * p.lda + (p.k - 1)) : 0u;
-    b_last = p.k > 0 ? load_value_uniform(B + (int64_t)(p.k - 1) * p.ldb + (p.n - 1)) : 0u;
-  }
-
-  // Issues the loads of stage kt into r.  The per-piece and per-stage parts of
-  // the offsets are wave-uniform (scalar offset operand).
-  __device__ __forceinline__ void issue(int kt, RawStage<G, false>& r) const {
-#pragma unroll
-    for (int i = 0; i < NA; ++i) r.a[i] = buffer_load16(a_rsrc, a_off, 2u * G::BK * (uint32_t)kt + i * a_step);
-    const int64_t skip = 2 * (int64_t)G::BK * kt * p.ldb;
-    const __amdgpu_buffer_rsrc_t b_rsrc = buffer_rsrc(b_tile + skip / 2, b_bytes - skip);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) r.b[i] = buffer_load16(b_rsrc, b_off, i * b_step);
-  }
-
-  // Writes stage kt, fetched into r, into LDS buffer s (16-byte stores).  Only
-  // the stage that holds k = K - 1 needs masking: A values at k >= K (the next
-  // row's head), B rows at k >= K, and the matrices' last values.
-  __device__ __forceinline__ void store(const RawStage<G, false>& r, int kt, uint16_t* lds, int s) const {
-    uint16_t* as = lds + s * G::STAGE + a_lds;
-    uint16_t* bs = lds + s * G::STAGE + G::A_STAGE + b_lds;
-    if (kt != last_stage) {
-#pragma unroll
-      for (int i = 0; i < NA; ++i) *reinterpret_cast<u32x4_t*>(as + i * A_LDS_STEP) = r.a[i];
-#pragma unroll
-      for (int i = 0; i < NB; ++i) *reinterpret_cast<u32x4_t*>(bs + i * B_LDS_STEP) = r.b[i];
-      return;
-    }
-    const int t = opaque_tid();
-    const int a_col = kt * G::BK + 8 * (t % APR);  // a thread's pieces share their columns
-    const int a_row = m0 + t / APR;
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      u32x4_t val = keep_values(r.a[i], p.k - a_col);
-      val = put_value(val, a_row + i * (T / APR) == p.m - 1 ? p.k - 1 - a_col : -1, a_last);
-      *reinterpret_cast<u32x4_t*>(as + i * A_LDS_STEP) = val;
-    }
-    const int b_col = n0 + 8 * (t % BPR);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int krow = kt * G::BK + t / BPR + i * (T / BPR);
-      const u32x4_t zero = {0u, 0u, 0u, 0u};
-      u32x4_t val = krow < p.k ? r.b[i] : zero;
-      val = put_value(val, krow == p.k - 1 ? p.n - 1 - b_col : -1, b_last);
-      *reinterpret_cast<u32x4_t*>(bs + i * B_LDS_STEP) = val;
-    }
-  }
-};
-
-template <class G>
-struct StageLoader<G, true> {
-  static constexpr int T = G::THREADS;
-  static constexpr int NA = G::A_PER_THREAD;
-  static constexpr int NB = G::B_PER_THREAD;
-  static constexpr int APR = G::BK / 8;
-  static constexpr int BPR = G::BN / 8;
 
   const gg_device_problem_desc& p;
   int tid;
@@ -533,14 +411,14 @@ struct StageLoader<G, true> {
     return edge_place(static_cast<const uint16_t*>(p.b), p.ldb, p.k, p.n, kt * G::BK + v / BPR, n0 + 8 * (v % BPR));
   }
 
-  __device__ __forceinline__ void issue(int kt, RawStage<G, true>& r) const {
+  __device__ __forceinline__ void issue(int kt, RawStage<G>& r) const {
 #pragma unroll
     for (int i = 0; i < NA; ++i) issue_piece_edge(a_edge(i, kt), r.a[i]);
 #pragma unroll
     for (int i = 0; i < NB; ++i) issue_piece_edge(b_edge(i, kt), r.b[i]);
   }
 
-  __device__ __forceinline__ void store(const RawStage<G, true>& r, int kt, uint16_t* lds, int s) const {
+  __device__ __forceinline__ void store(const RawStage<G>& r, int kt, uint16_t* lds, int s) const {
     const int t = opaque_tid();
     uint16_t* as = lds + s * G::STAGE;
     uint16_t* bs = as + G::A_STAGE;
@@ -615,7 +493,6 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 // once its loads have landed.
 template <class G>
 struct DmaLoader {
-  static_assert(G::A_SWIZZLED, "a load into LDS writes unpadded rows");
   static constexpr int T = G::THREADS;
   static constexpr int WAVES = T / kWave;
   static constexpr int NA = G::A_PER_THREAD;

@@ -56,7 +56,7 @@ template <class G>
 struct PhasedLoader {
   static constexpr int UNIT = 128 * 64;  // values of a unit
   static constexpr int A0 = 0, B0 = UNIT, B1 = 2 * UNIT, A1 = 3 * UNIT, PARITY = 4 * UNIT;
-  static_assert(G::BM == 256 && G::BN == 256 && G::BK == 64 && G::THREADS == 512 && G::A_SWIZZLED, "the full work tile");
+  static_assert(G::BM == 256 && G::BN == 256 && G::BK == 64 && G::THREADS == 512, "the full work tile");
   static_assert(2 * PARITY <= G::LDS_HALVES, "two stages");
   static constexpr int WAVES = 8;
   static constexpr int LOADS = 2;  // load instructions per unit and wave

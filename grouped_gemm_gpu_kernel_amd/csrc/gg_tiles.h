@@ -2,12 +2,12 @@
 //
 // The MFMA path loads its stages straight into LDS and multiplies them a phase
 // behind the fragment reads (run_k_loop_halves here, run_k_loop_phased in
-// gg_phased.h for the full 256 x 256 work tile).  The FMA path and the 64-bit
-// addressing forms stage through registers: each K stage is read from global
-// memory into registers while the previous stage, held in LDS, is being
-// multiplied; the registers are then written to the other LDS buffer and one
-// barrier ends the stage.  The reference's equivalents are compute_gemm_tile_tensor_core and
-// compute_gemm_tile_simt (src/grouped_gemm.cu:373-626); the k-loop structure,
+// gg_phased.h for the full 256 x 256 work tile), as the FMA path does
+// (run_k_loop_fma).  The 64-bit addressing forms stage through registers: each
+// K stage is read from global memory into registers while the previous stage,
+// held in LDS, is being multiplied; the registers are then written to the
+// other LDS buffer and one barrier ends the stage.  The reference's
+// equivalents are compute_gemm_tile_tensor_core and compute_gemm_tile_simt (src/grouped_gemm.cu:373-626); the k-loop structure,
 // register blocking and LDS layout here are gfx950's own.
 #pragma once
 
@@ -16,7 +16,7 @@
 
 namespace gg {
 
-// Runs the staged k-loop of one tile: compute(stage_pointer) is called once
+// Runs the staged k-loop of one tile in the 64-bit addressing form: compute(stage_pointer) is called once
 // per stage with that stage's LDS buffer, and on_start() once, by every
 // thread, after the first loads are on their way (the persistent scheduler
 // requests its next tile there, so that the request's latency overlaps this
@@ -34,7 +34,7 @@ namespace gg {
 // runs whole groups of DEPTH steps with no branch; the last steps of a tile
 // are guarded.  The body is unrolled DEPTH times so that every register set
 // is addressed statically.
-template <class G, bool WIDE, class Compute, class OnStart, class Stamps>
+template <class G, class Compute, class OnStart, class Stamps>
 __device__ __forceinline__ void run_k_loop(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
                                            Compute&& compute, OnStart&& on_start, const Stamps& stamps) {
   constexpr int D = G::DEPTH;
@@ -43,8 +43,8 @@ __device__ __forceinline__ void run_k_loop(const gg_device_problem_desc& p, int 
     on_start();
     return;
   }
-  const StageLoader<G, WIDE> loader(p, m0, n0);
-  RawStage<G, WIDE> ring[D];
+  const StageLoader<G> loader(p, m0, n0);
+  RawStage<G> ring[D];
 #pragma unroll
   for (int s = 0; s < D - 1; ++s) loader.issue(s, ring[s]);
   on_start();  // the compiler's waits count the request like any other load
@@ -243,6 +243,52 @@ __device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& 
   if constexpr (!std::is_same_v<Stamps, NoStamps>) phase_barrier();
 }
 
+// The FMA path's k-loop with stage loads straight into LDS: compute(stage,
+// first k) once per stage.  A stage's buffer is asked for stage t + 2 when
+// every wave has multiplied stage t, so no load waits in registers, and one
+// copy of the multiplying code serves every stage.  Staged through a ring of
+// three register sets the code came in five copies (40 KB) and a CU held two
+// workgroups of 64 x 64 tiles; it holds four with 32 KB of LDS each.  256 problems of
+// 16 to 256 in each dimension (893 tiles): 31.2 -> 29.3 us, with FmaTile's
+// vector epilogue 26.0.  A launch like that is bound by each tile's own chain:
+// a 64 x 64 tile 256 deep takes 6.8 us of FMAs, all tiles together 5.9 us of the chip.
+template <class G, class Compute, class OnStart, class Stamps>
+__device__ __forceinline__ void run_k_loop_fma(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
+                                               Compute&& compute, OnStart&& on_start, const Stamps& stamps) {
+  using L = DmaLoader<G>;
+  constexpr int NBUF = G::BUFFERS;
+  constexpr int LOADS = L::LOADS;
+  static_assert(NBUF == 2, "the waits below are those of two buffers");
+  const int nk = (p.k + G::BK - 1) / G::BK;
+  if (nk <= 0) {
+    on_start();
+    return;
+  }
+  const L loader(p, m0, n0);
+  loader.issue(0, lds);
+  if (nk > 1) loader.issue(1, lds + G::STAGE);
+  const bool extra = __builtin_amdgcn_readfirstlane(on_start() ? 1 : 0) != 0;
+#pragma unroll 1
+  for (int t = 0; t < nk; ++t) {
+    uint16_t* const stage = lds + (t & 1) * G::STAGE;
+    // In flight behind the loads of stage t: those of stage t + 1 and, at the start, the request.
+    if (t + 1 == nk) {
+      if (t == 0 && extra) wait_vmcnt<1>(); else wait_vmcnt<0>();
+    } else {
+      if (t == 0 && extra) wait_vmcnt<LOADS + 1>(); else wait_vmcnt<LOADS>();
+    }
+    if (t == 0) stamps.mark(GGK_PHASE_FIRST_STAGE);
+    if (t == loader.last_stage) loader.fix_last_stage(t, stage);
+    stage_barrier();
+    if (t == 0) stamps.mark(GGK_PHASE_K_LOOP);
+    compute(stage, t * G::BK);
+    if (t + 2 < nk) {
+      stage_barrier();
+      loader.issue(t + 2, stage);
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // MFMA tile: v_mfma_f32_16x16x32_f16, (BM/WM) x (BN/64) waves, each owning a
 // WM x 64 block of D held as (WM/16) x 4 16x16 accumulators.  Per product the
@@ -369,7 +415,7 @@ struct MfmaTile {
       if (live) compute_stage(stage, lane, wm, wn, acc);
     };
     if constexpr (WIDE) {
-      run_k_loop<G, WIDE>(p, m0, n0, lds, compute, on_start, stamps);
+      run_k_loop<G>(p, m0, n0, lds, compute, on_start, stamps);
     } else if constexpr (PHASED) {
       run_k_loop_phased<G>(p, m0, n0, lds, wm, wn, acc, on_start, stamps);
     } else {
@@ -549,7 +595,8 @@ struct MfmaTile {
 // tm*RM .. tm*RM+RM-1 and columns tn*RN .. tn*RN+RN-1 of the macro-tile, with
 // RM = BM/16, RN = BN/16 float32 accumulators.  Per 8-deep k slice a thread
 // reads one 16-byte piece of each of its A rows and one RN-wide piece of each
-// B row from LDS, then issues RM*RN*8 fused multiply-adds in ascending k.
+// B row from LDS (while the slice before is multiplied), then issues RM*RN*8
+// fused multiply-adds in ascending k.
 // Used when MFMA is not requested (use_tensor_cores = false).
 // ---------------------------------------------------------------------------
 template <class G>
@@ -559,38 +606,48 @@ struct FmaTile {
   static_assert(RN == 4 || RN == 8, "column block must be one or two LDS chunks");
   static_assert(G::THREADS == 256, "16 x 16 thread grid");
 
-  __device__ __forceinline__ static void compute_stage(const uint16_t* stage, int krem, int tm, int tn,
-                                                       float (&acc)[RM][RN]) {
-    const uint16_t* as = stage;
-    const uint16_t* bs = stage + G::A_STAGE;
+  // The operands of an 8-deep slice of a stage: RM rows of A, 8 k-rows of B.
+  using brow_t = std::conditional_t<RN == 4, half4_t, half8_t>;
+  struct Slice {
+    half8_t a[RM];
+    brow_t b[8];
+  };
+  __device__ __forceinline__ static void load_slice(const uint16_t* stage, int k8, int tm, int tn, Slice& s) {
 #pragma unroll
-    for (int k8 = 0; k8 < G::BK / 8; ++k8) {
-      if (k8 * 8 >= krem) break;
-      half8_t av[RM];
+    for (int i = 0; i < RM; ++i) s.a[i] = *reinterpret_cast<const half8_t*>(stage + G::a_piece(tm * RM + i, k8));
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+      s.b[kk] = *reinterpret_cast<const brow_t*>(stage + G::A_STAGE + G::b_chunk(k8 * 8 + kk, tn * RN));
+    }
+  }
+  __device__ __forceinline__ static void multiply_slice(const Slice& s, float (&acc)[RM][RN]) {
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
 #pragma unroll
       for (int i = 0; i < RM; ++i) {
-        av[i] = *reinterpret_cast<const half8_t*>(as + G::a_piece(tm * RM + i, k8));
+        const float a = (float)s.a[i][kk];
+#pragma unroll
+        for (int j = 0; j < RN; ++j) acc[i][j] = __builtin_fmaf(a, (float)s.b[kk][j], acc[i][j]);
       }
-#pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
-        const uint16_t* brow = bs + G::b_chunk(k8 * 8 + kk, tn * RN);
-        float bv[RN];
-        if constexpr (RN == 4) {
-          const half4_t h = *reinterpret_cast<const half4_t*>(brow);
-#pragma unroll
-          for (int j = 0; j < RN; ++j) bv[j] = (float)h[j];
-        } else {
-          const half8_t h = *reinterpret_cast<const half8_t*>(brow);
-#pragma unroll
-          for (int j = 0; j < RN; ++j) bv[j] = (float)h[j];
-        }
-#pragma unroll
-        for (int i = 0; i < RM; ++i) {
-          const float a = (float)av[i][kk];
-#pragma unroll
-          for (int j = 0; j < RN; ++j) acc[i][j] = __builtin_fmaf(a, bv[j], acc[i][j]);
-        }
-      }
+    }
+  }
+  __device__ __forceinline__ static void compute_stage(const uint16_t* stage, int krem, int tm, int tn,
+                                                       float (&acc)[RM][RN]) {
+    const int slices = krem >= G::BK ? G::BK / 8 : (krem + 7) / 8;
+    // The next slice is read while this one is multiplied (past the last: one that is not used).
+    Slice even, odd;
+    load_slice(stage, 0, tm, tn, even);
+#pragma unroll 1
+    for (int k8 = 0; k8 < slices; k8 += 2) {
+      load_slice(stage, k8 + 1, tm, tn, odd);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply_slice(even, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      if (k8 + 1 == slices) break;
+      load_slice(stage, (k8 + 2) % (G::BK / 8), tm, tn, even);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply_slice(odd, acc);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 
@@ -611,34 +668,95 @@ struct FmaTile {
 #pragma unroll
       for (int j = 0; j < RN; ++j) acc[i][j] = 0.0f;
 
-    int kt = 0;
-    run_k_loop<G, WIDE>(p, m0, n0, lds, [&](const uint16_t* stage) {
-      if (active) compute_stage(stage, p.k - kt * G::BK, tm, tn, acc);
-      ++kt;
-    }, on_start, stamps);
+    // The thread's part of C, as 16-byte vectors through a buffer resource from
+    // the wave's first row (vectors past N read as zero), asked for before the
+    // k-loop's loads.  Read and written as dwords after the k-loop: 29.3 us
+    // where this takes 26.0 (256 problems of 16 to 256 in each dimension).
+    const bool use_c = p.c != nullptr && p.beta != 0.0f;
+    const int r0 = __builtin_amdgcn_readfirstlane(m0 + (tid / kWave) * 4 * RM);
+    const int row_lane = ((tid & (kWave - 1)) >> 4) * RM;
+    floatx4_t early[RM][RN / 4];
+#pragma unroll
+    for (int i = 0; i < RM; ++i)
+#pragma unroll
+      for (int v = 0; v < RN / 4; ++v) early[i][v] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    if (!WIDE && use_c && active) {
+      const __amdgpu_buffer_rsrc_t crs =
+          buffer_rsrc(p.c + ((int64_t)r0 * p.ldc + n0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldc + (p.n - n0)));
+#pragma unroll
+      for (int i = 0; i < RM; ++i)
+#pragma unroll
+        for (int v = 0; v < RN / 4; ++v) {
+          const int col = tn * RN + 4 * v;
+          const uint32_t off = n0 + col < p.n ? 4u * ((uint32_t)(row_lane + i) * (uint32_t)p.ldc + (uint32_t)col)
+                                              : DmaLoader<G>::kOutOfRange;
+          early[i][v] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(crs, (int)off, 0, 0));
+        }
+    }
+
+    if constexpr (WIDE) {
+      int kt = 0;
+      run_k_loop<G>(p, m0, n0, lds, [&](const uint16_t* stage) {
+        if (active) compute_stage(stage, p.k - kt * G::BK, tm, tn, acc);
+        ++kt;
+      }, on_start, stamps);
+    } else {
+      run_k_loop_fma<G>(p, m0, n0, lds, [&](const uint16_t* stage, int k0) {
+        if (active) compute_stage(stage, p.k - k0, tm, tn, acc);
+      }, on_start, stamps);
+    }
     after_k_loop();
 
     if (!active) {
       stamps.wave_done();
       return;
     }
-    const bool use_c = p.c != nullptr && p.beta != 0.0f;
-    g_cf32_t* cptr = (g_cf32_t*)p.c;
-    g_f32_t* dptr = (g_f32_t*)p.d;
+    if constexpr (WIDE) {
+      g_cf32_t* cptr = (g_cf32_t*)p.c;
+      g_f32_t* dptr = (g_f32_t*)p.d;
 #pragma unroll
-    for (int i = 0; i < RM; ++i) {
-      const int row = m0 + tm * RM + i;
-      if (row >= p.m) continue;
-      float cv[RN];
+      for (int i = 0; i < RM; ++i) {
+        const int row = m0 + tm * RM + i;
+        if (row >= p.m) continue;
+        float cv[RN];
 #pragma unroll
-      for (int j = 0; j < RN; ++j) {
-        const int col = n0 + tn * RN + j;
-        cv[j] = (use_c && col < p.n) ? cptr[(int64_t)row * p.ldc + col] : 0.0f;
+        for (int j = 0; j < RN; ++j) {
+          const int col = n0 + tn * RN + j;
+          cv[j] = (use_c && col < p.n) ? cptr[(int64_t)row * p.ldc + col] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < RN; ++j) {
+          const int col = n0 + tn * RN + j;
+          if (col < p.n) dptr[(int64_t)row * p.ldd + col] = epilogue_value(acc[i][j], cv[j], p.alpha, use_c ? p.beta : 0.0f);
+        }
       }
+    } else {
+      const __amdgpu_buffer_rsrc_t drs =
+          buffer_rsrc(p.d + ((int64_t)r0 * p.ldd + n0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldd + (p.n - n0)));
 #pragma unroll
-      for (int j = 0; j < RN; ++j) {
-        const int col = n0 + tn * RN + j;
-        if (col < p.n) dptr[(int64_t)row * p.ldd + col] = epilogue_value(acc[i][j], cv[j], p.alpha, use_c ? p.beta : 0.0f);
+      for (int i = 0; i < RM; ++i) {
+        const int row = row_lane + i;
+        if (r0 + row >= p.m) continue;
+#pragma unroll
+        for (int v = 0; v < RN / 4; ++v) {
+          const int col = tn * RN + 4 * v;
+          const int ncol = p.n - (n0 + col);
+          const uint32_t off = 4u * ((uint32_t)row * (uint32_t)p.ldd + (uint32_t)col);
+          floatx4_t out;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            out[e] = epilogue_value(acc[i][4 * v + e], early[i][v][e], p.alpha, use_c ? p.beta : 0.0f);
+          }
+          if (ncol >= 4) {
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) int, out), drs,
+                                                   (int)off, 0, 0);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+              if (e < ncol) __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(out[e]), drs, (int)(off + 4 * e), 0, 0);
+            }
+          }
+        }
       }
     }
     stamps.wave_done();
