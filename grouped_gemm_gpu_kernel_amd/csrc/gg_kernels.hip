@@ -167,6 +167,29 @@ __device__ __forceinline__ int chunk_bound(const GroupedArgs& args, int split, i
   return b;
 }
 
+// The index a workgroup without a fixed tile computes when the launch has no
+// more work tiles than workgroups (-1: none).  Chunks differ in size, so some
+// hold more indices than workgroups start there and others fewer: the spare
+// workgroups, counted over the chunks, take the indices left over, counted the
+// same way, one each.  No counter is read, asked or reset: 256 problems of 893
+// FMA tiles 26.0 -> 21.9 us, where a sixth of the workgroups had to ask for
+// their first tile and every one waited for its retirement.
+__device__ __forceinline__ int spare_tile(const GroupedArgs& args, int split, int grid, int home) {
+  int spare = (int)blockIdx.x / kChunks;  // spare workgroups before this one
+  for (int c = 0; c <= home; ++c) {
+    const int size = chunk_bound(args, split, c + 1) - chunk_bound(args, split, c);
+    const int slots = fixed_slots(c, grid);
+    spare += c == home ? -size : (slots > size ? slots - size : 0);
+  }
+  for (int c = 0; c < kChunks; ++c) {
+    const int from = chunk_bound(args, split, c) + fixed_slots(c, grid);
+    const int left = chunk_bound(args, split, c + 1) - from;
+    if (spare < left) return from + spare;
+    spare -= left > 0 ? left : 0;
+  }
+  return -1;
+}
+
 // Index of the problem that owns index t: the number of problems p with
 // offsets[p + 1] <= t, i.e. upper_bound over offsets[1..count] -- the same
 // function as find_problem_by_tile (src/grouped_gemm.cu:219-234), here over
@@ -277,17 +300,21 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
       kSplits && args.header != nullptr && 2 * ((const_int_ptr)args.header)[1] <= grid ? 1 : 0;
   int t = chunk_bound(args, split, home) + (int)blockIdx.x / kChunks;
   const bool fixed = t < chunk_bound(args, split, home + 1);
+  // At most one work tile per workgroup: every tile is fixed (spare_tile).
+  const bool one_each = chunk_bound(args, split, kChunks) - chunk_bound(args, split, 0) <= grid;
   // Wave 0: the chunks with indices beyond the fixed first tiles.  When there
   // is none, no counter is touched and none needs resetting.
   uint32_t counted = 0;
-  if (wave0) {
+  if (wave0 && !one_each) {
     load_schedule(args, split, s_schedule);
     counted = counted_chunks(s_schedule, grid);
   }
 
   int visit = 0;  // wave 0
   int parity = 0;
-  if (!fixed) {
+  if (!fixed && one_each) {
+    t = spare_tile(args, split, grid, home);
+  } else if (!fixed) {
     // No fixed tile for this workgroup (its chunk is smaller than its share
     // of the grid): claim one now.
     if (wave0) {
