@@ -535,8 +535,8 @@ def _stats(v) -> str:
     return f"dispatches {len(v)}  mean {sum(v) / len(v):.6g}  min {min(v):.6g}  max {max(v):.6g}"
 
 
-MFMA_CYCLES = 32        # v_mfma_f32_32x32x16_f16: cycles a SIMD is busy per instruction
-MFMA_MACS = 32 * 32 * 16
+MFMA_CYCLES = 16        # v_mfma_f32_16x16x32_f16: cycles a SIMD is busy per instruction
+MFMA_MACS = 16 * 16 * 32
 SIMDS_PER_CU = 4
 XCDS = 8
 CUS = 256
@@ -546,8 +546,8 @@ def _derived(metrics, workload) -> list:
     """Ratios of the counters of one sort mode (means per dispatch):
       mfma_busy        SQ_VALU_MFMA_BUSY_CYCLES / (4 SIMDs x SQ_BUSY_CU_CYCLES): share of the SIMD
                        cycles of busy CUs spent in MFMA;
-      mfma_executed    SQ_VALU_MFMA_BUSY_CYCLES / 32 cycles per 32x32x16 MFMA, against the
-                       workload's useful MFMAs (sum m n k / 16384): padding of partial tiles;
+      mfma_executed    SQ_VALU_MFMA_BUSY_CYCLES / 16 cycles per 16x16x32 MFMA, against the
+                       workload's useful MFMAs (sum m n k / 8192): padding of partial tiles;
       l2_hit           TCC_HIT / (TCC_HIT + TCC_MISS);
       lds_bank_conflict  SQ_LDS_BANK_CONFLICT / SQ_LDS_IDX_ACTIVE (cycles);
       clock_ghz        GRBM_GUI_ACTIVE / 8 XCDs / the dispatch's duration (when traced);
