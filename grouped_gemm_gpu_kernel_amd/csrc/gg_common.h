@@ -22,6 +22,10 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kWave = 64;
 
+// Bytes every LDS stage starts on a multiple of: fragment addresses select
+// k-halves and column blocks by XOR on address bits 5 and 6.
+constexpr int kStageAlign = 128;
+
 // Geometry of one kernel's work tile.  BM x BN is the block of D a workgroup
 // computes per claim; BK is the depth of one LDS stage; THREADS is the
 // workgroup size.  The reference's macro-tile (cta_m x cta_n,
@@ -81,7 +85,7 @@ struct Geometry {
   // so rows k..k+3 (k a multiple of 4) land on 4 different 64-byte bank
   // windows, and with 4 by 32 bytes, so rows k and k + 8 take different halves
   // of a window.
-  __device__ static __forceinline__ int b_swizzle(int k) {
+  __host__ __device__ static constexpr int b_swizzle(int k) {
     if constexpr (BN == 64) {
       return 8 * ((k >> 1) & 1);
     } else {
@@ -90,15 +94,41 @@ struct Geometry {
   }
   // Element offset, within a B stage, of the 4-value chunk that holds (k, n)
   // for n a multiple of 4.
-  __device__ static __forceinline__ int b_chunk(int k, int n) { return k * SB + 4 * ((n >> 2) ^ b_swizzle(k)); }
+  __host__ __device__ static constexpr int b_chunk(int k, int n) { return k * SB + 4 * ((n >> 2) ^ b_swizzle(k)); }
 
   // A: rows that share a 256-byte bank window (row / RPW equal) get distinct
   // piece positions; RPW = 256 / (2 BK) rows per window.
   static constexpr int A_RPW = 128 / BK;
-  __device__ static __forceinline__ int a_swizzle(int row) { return (row / A_RPW) & (APR - 1); }
+  __host__ __device__ static constexpr int a_swizzle(int row) { return (row / A_RPW) & (APR - 1); }
   // Element offset, within an A stage, of the 16-byte piece c (values 8c ..
   // 8c + 7 of the stage's k range) of a row.
-  __device__ static __forceinline__ int a_piece(int row, int c) { return row * SA + 8 * (c ^ a_swizzle(row)); }
+  __host__ __device__ static constexpr int a_piece(int row, int c) { return row * SA + 8 * (c ^ a_swizzle(row)); }
+
+  // LDS byte addresses of operand fragments for the k-loops on loads straight
+  // into LDS (64-deep stages).  `at` is the address of the lane's fragment of
+  // k-half 0 (A, a 16-byte piece) or of column block 0 (B, an 8-byte chunk),
+  // and `values` whole rows further on.  The k-half selects bit 6 of A's
+  // address, the 16-column block bits 5 and 6 of B's (the swizzles are XORs):
+  // bits of the offset in the stage only as long as every stage, and the LDS
+  // array itself, starts on a multiple of kStageAlign.
+  __host__ __device__ static constexpr uint32_t a_fragment(uint32_t at, int k_half, int values) {
+    static_assert(BK == 64 && (2 * A_STAGE) % kStageAlign == 0 && (2 * STAGE) % kStageAlign == 0 &&
+                      (2 * SA) % kStageAlign == 0,
+                  "bit 6 of an A address is the k-half alone");
+    return (at ^ (uint32_t)(64 * k_half)) + 2u * (uint32_t)values;
+  }
+  __host__ __device__ static constexpr uint32_t b_fragment(uint32_t at, int block, int values) {
+    static_assert((2 * A_STAGE) % kStageAlign == 0 && (2 * STAGE) % kStageAlign == 0 && (2 * SB) % kStageAlign == 0,
+                  "bits 5 and 6 of a B address are the column block alone");
+    return (at ^ (uint32_t)(32 * block)) + 2u * (uint32_t)values;
+  }
+};
+
+// The stage buffers of a kernel in LDS.  The type carries their alignment, so
+// that it does not depend on what else a kernel declares in LDS.
+template <int N>
+struct alignas(kStageAlign) StageRing {
+  uint16_t values[N];
 };
 
 #ifndef GG_STAGE_K

@@ -273,7 +273,7 @@ template <int V, int PATH, bool TRACED, bool WIDE>
 __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
   using S = KernelShape<V, PATH>;
   using G = typename S::G;
-  __shared__ __attribute__((aligned(16))) uint16_t lds[KernelLds<S>::HALVES];
+  __shared__ StageRing<KernelLds<S>::HALVES> lds;
   __shared__ int s_claim[2];
   __shared__ int s_schedule[kChunks + 1];
 
@@ -464,7 +464,7 @@ template <int V, int PATH, bool WIDE>
 __global__ GG_KERNEL_ATTRS(V, PATH) void gg_single_kernel(gg_device_problem_desc p) {
   using S = KernelShape<V, PATH>;
   using G = typename S::G;
-  __shared__ __attribute__((aligned(16))) uint16_t lds[KernelLds<S>::HALVES];
+  __shared__ StageRing<KernelLds<S>::HALVES> lds;
   const int t = blockIdx.x;
   const int wtn = work_tiles_n<S::TM, S::TN>(p);
   const int wtm = (p.tiles_m + S::TM - 1) / S::TM;

@@ -182,17 +182,16 @@ __device__ __forceinline__ void run_k_loop_phased(const gg_device_problem_desc& 
       lds_address(lds) + 2u * (uint32_t)G::b_chunk(8 * g + (j >> 2), wn * 64 + 4 * (j & 3));
 
   // Fragment read r (0..7) of the unit at offset `unit` (values) of a stage at
-  // byte offset `stage` of the ring.  The k-step selects bit 6 of A's address,
-  // the column block bits 5 and 6 of B's (the swizzles are XORs).
+  // byte offset `stage` of the ring.
+  static_assert((2 * L::UNIT) % kStageAlign == 0, "a unit keeps the address bits that select a fragment");
   auto read_a = [&](int half, int unit, uint32_t stage, int r) {
     const int fm = r & 3, s = r >> 2;
-    const uint32_t at = (a_lane + stage) ^ (uint32_t)(64 * s);
-    a[half][fm][s] = *(const GG_LDS half8_t*)(uintptr_t)(at + 2u * (uint32_t)(unit + fm * 16 * G::SA));
+    a[half][fm][s] = *(const GG_LDS half8_t*)(uintptr_t)G::a_fragment(a_lane + stage, s, unit + fm * 16 * G::SA);
   };
   short4_t b_lo;
   auto read_b = [&](int half, int unit, uint32_t stage, int r) {
     const int fn = r >> 1;
-    const uint32_t at = ((b_lane + stage) ^ (uint32_t)(32 * fn)) + 2u * (uint32_t)unit;
+    const uint32_t at = G::b_fragment(b_lane + stage, fn, unit);
     if ((r & 1) == 0) {
       b_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GG_LDS short4_t*)(uintptr_t)at);
     } else {

@@ -136,13 +136,12 @@ __device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& 
   const uint32_t b_lane = lds_address(lds) + 2u * (uint32_t)(G::A_STAGE + G::b_chunk(8 * g + (j >> 2),
                                                                                       wn * 64 + 4 * (j & 3)));
   // Fragment read r (0..FM + 7) of k-half h of the stage at byte offset `at`
-  // of the ring: the k-half selects bit 6 of A's address, the column block bits
-  // 5 and 6 of B's (the swizzles are XORs).
+  // of the ring.
   short4_t b_lo;
   auto read = [&](int h, uint32_t at, int r) {
     if (r < 8) {
       const int fn = r >> 1;
-      const uint32_t addr = ((b_lane + at) ^ (uint32_t)(32 * fn)) + (uint32_t)(64 * h) * G::SB;
+      const uint32_t addr = G::b_fragment(b_lane + at, fn, 32 * h * G::SB);
       if ((r & 1) == 0) {
         b_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((GG_LDS short4_t*)(uintptr_t)addr);
       } else {
@@ -151,7 +150,7 @@ __device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& 
       }
     } else {
       const int fm = r - 8;
-      a[h][fm] = *(const GG_LDS half8_t*)(uintptr_t)(((a_lane + at) ^ (uint32_t)(64 * h)) + (uint32_t)(32 * fm) * G::SA);
+      a[h][fm] = *(const GG_LDS half8_t*)(uintptr_t)G::a_fragment(a_lane + at, h, 16 * fm * G::SA);
     }
   };
   // The MFMAs of k-half h, among them the reads of the next half and
@@ -787,9 +786,10 @@ struct KernelLds<S, true> {
 // problem selects (KernelShape::CLASSES), else in the kernel's own form.  The
 // class is uniform across the workgroup (scalar descriptor and origin).
 template <class S, int PATH, bool WIDE, class OnStart, class AfterKLoop, class Stamps = NoStamps>
-__device__ __forceinline__ void run_work_tile(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
-                                              OnStart&& on_start, AfterKLoop&& after_k_loop,
-                                              const Stamps& stamps = Stamps{}) {
+__device__ __forceinline__ void run_work_tile(const gg_device_problem_desc& p, int m0, int n0,
+                                              StageRing<KernelLds<S>::HALVES>& ring, OnStart&& on_start,
+                                              AfterKLoop&& after_k_loop, const Stamps& stamps = Stamps{}) {
+  uint16_t* const lds = ring.values;
   if constexpr (PATH == GGK_PATH_MFMA && !WIDE && S::CLASSES) {
     const bool rows = p.m - m0 <= S::G::BM / 2;
     const bool cols = p.n - n0 <= S::G::BN / 2;
