@@ -369,11 +369,11 @@ Schedule plan_schedule(const std::vector<DeviceProblemDesc>& problems, const std
 // scheduler state, each part starting on a 256-byte boundary (the state's
 // counters then sit on 128-byte lines of their own).  Launches read it until
 // they end, so it is rewritten or freed only after the last launch's event
-// (recorded on that launch's stream) has completed.  A launch captured into a
-// graph records no event, and the graph may be replayed on any stream at any
-// later time: once a launch was captured, every wait is for the whole device
-// instead, until the allocation is released (the device must then not be
-// capturing).
+// (signalled by the launch or recorded behind it, see tracked_launch) has
+// completed.  A launch captured into a graph records no event, and the graph
+// may be replayed on any stream at any later time: once a launch was captured,
+// every wait is for the whole device instead, until the allocation is released
+// (the device must then not be capturing).
 struct DeviceBuffer {
   void* base = nullptr;
   size_t capacity = 0;  // bytes
@@ -381,6 +381,9 @@ struct DeviceBuffer {
   hipEvent_t last_launch = nullptr;
   bool launched = false;  // an event was recorded since the last wait
   bool captured = false;  // a launch was captured since the allocation was made
+  hipStream_t recorded_stream = nullptr;  // where the event was last recorded behind a launch
+  int carried = kCarriedLaunches;         // launches since then, all on that stream, that signalled it themselves
+  static constexpr int kCarriedLaunches = 63;
 
   static size_t round256(size_t x) { return (x + 255) / 256 * 256; }
 
@@ -396,11 +399,34 @@ struct DeviceBuffer {
     return ggk_event_synchronize(last_launch);
   }
 
-  // Notes a launch whose completion signals last_launch (GGK_LAUNCH_RECORDED)
-  // or that was captured (GGK_LAUNCH_CAPTURED).
-  void note_launch(int recorded) {
-    if (recorded == GGK_LAUNCH_RECORDED) launched = true;
+  // Makes a launch on `stream` with launch(done, &recorded) and has its
+  // completion signal last_launch: the launch carries the event itself, or the
+  // event is recorded behind it.  Carrying it saves the stream a packet (2.5 us
+  // a launch), but the HIP runtime keeps such a launch's host object (1.4 KB)
+  // until it has processed a record on that stream, or a wait that found the
+  // stream busy; a query, a copy or an allocation does not let go of it, and
+  // 80,000 launches of a loop without waits kept 111 MB.  So the event is
+  // recorded behind the first launch on a stream and behind every 64th after
+  // it: the loop then keeps 2.8 MB at most (4.5 MB with a record behind every
+  // launch), for 0.04 us a launch, and building a plan of 16 problems after
+  // 2,000 passes takes 0.52 ms again instead of 0.68.  (The per-thread stream's
+  // handle stands for a stream of each thread, so there every launch counts as
+  // the first.)  can_carry: whether launch takes the event at all.
+  template <class Launch>
+  hipError_t tracked_launch(hipStream_t stream, bool can_carry, Launch&& launch) {
+    const bool carry = can_carry && last_launch != nullptr && carried < kCarriedLaunches &&
+                       stream == recorded_stream && stream != hipStreamPerThread;
+    int recorded = 0;
+    hipError_t status = launch(carry ? last_launch : nullptr, &recorded);
+    if (status != hipSuccess || last_launch == nullptr) return status;
+    if (!carry) status = ggk_event_record_launch(last_launch, stream, &recorded);
+    if (recorded == GGK_LAUNCH_RECORDED) {
+      launched = true;
+      carried = carry ? carried + 1 : 0;
+      recorded_stream = stream;
+    }
     if (recorded == GGK_LAUNCH_CAPTURED) captured = true;
+    return status;
   }
 
   // At least `bytes` on the current device, reusing the allocation when it is
@@ -441,6 +467,7 @@ struct DeviceBuffer {
     last_launch = nullptr;
     launched = false;
     captured = false;
+    carried = kCarriedLaunches;
   }
 };
 
@@ -923,14 +950,12 @@ hipError_t GroupedGemmExecutor::run(hipStream_t stream) const {
   if (impl_ == nullptr) return hipErrorInvalidDevicePointer;
   if (impl_->failed) return hipErrorInvalidValue;
   if (impl_->total_tiles == 0 || impl_->problem_count == 0) return hipSuccess;
-  int recorded = 0;
-  const hipError_t status = ggk_launch_grouped_done(
-      impl_->variant, impl_->path, impl_->addressing, impl_->d_problems, impl_->d_ints + impl_->problem_count + 1,
-      impl_->d_ints + 2 * (impl_->problem_count + 1), impl_->d_work_table(), impl_->problem_count,
-      impl_->launch_total, impl_->d_state, impl_->launch_bounds.data(), impl_->grid_ctas,
-      impl_->buffer.last_launch, &recorded, stream);
-  if (status == hipSuccess) impl_->buffer.note_launch(recorded);
-  return status;
+  return impl_->buffer.tracked_launch(stream, true, [&](hipEvent_t done, int* recorded) {
+    return ggk_launch_grouped_done(
+        impl_->variant, impl_->path, impl_->addressing, impl_->d_problems, impl_->d_ints + impl_->problem_count + 1,
+        impl_->d_ints + 2 * (impl_->problem_count + 1), impl_->d_work_table(), impl_->problem_count,
+        impl_->launch_total, impl_->d_state, impl_->launch_bounds.data(), impl_->grid_ctas, done, recorded, stream);
+  });
 }
 
 hipError_t GroupedGemmExecutor::run_traced(int* d_tile_map, long long* d_wg_clock, hipStream_t stream,
@@ -938,16 +963,13 @@ hipError_t GroupedGemmExecutor::run_traced(int* d_tile_map, long long* d_wg_cloc
   if (impl_ == nullptr) return hipErrorInvalidDevicePointer;
   if (impl_->failed) return hipErrorInvalidValue;
   if (impl_->total_tiles == 0 || impl_->problem_count == 0) return hipSuccess;
-  hipError_t status = ggk_launch_grouped_traced(
-      impl_->variant, impl_->path, impl_->addressing, impl_->d_problems, impl_->d_ints,
-      impl_->d_ints + impl_->problem_count + 1, impl_->d_ints + 2 * (impl_->problem_count + 1), impl_->d_work_table(),
-      impl_->problem_count, impl_->launch_total, impl_->d_state, impl_->launch_bounds.data(), impl_->grid_ctas, d_tile_map,
-      d_wg_clock, d_tile_phases, stream);
-  if (status != hipSuccess || impl_->buffer.last_launch == nullptr) return status;
-  int recorded = 0;
-  status = ggk_event_record_launch(impl_->buffer.last_launch, stream, &recorded);
-  impl_->buffer.note_launch(recorded);
-  return status;
+  return impl_->buffer.tracked_launch(stream, false, [&](hipEvent_t, int*) {
+    return ggk_launch_grouped_traced(
+        impl_->variant, impl_->path, impl_->addressing, impl_->d_problems, impl_->d_ints,
+        impl_->d_ints + impl_->problem_count + 1, impl_->d_ints + 2 * (impl_->problem_count + 1),
+        impl_->d_work_table(), impl_->problem_count, impl_->launch_total, impl_->d_state,
+        impl_->launch_bounds.data(), impl_->grid_ctas, d_tile_map, d_wg_clock, d_tile_phases, stream);
+  });
 }
 
 int GroupedGemmExecutor::problem_count() const { return impl_ != nullptr ? impl_->problem_count : 0; }
@@ -1288,17 +1310,16 @@ hipError_t MoeGroupedGemm::build(const MoeLayout& layout, const KernelConfig& co
 hipError_t MoeGroupedGemm::run(const int* d_counts, hipStream_t stream) const {
   if (impl_ == nullptr || impl_->d_problems == nullptr || impl_->variant < 0) return hipErrorInvalidDevicePointer;
   if (d_counts == nullptr) return hipErrorInvalidDevicePointer;
-  hipError_t status = ggk_moe_prepare(impl_->variant, impl_->path, &impl_->layout, d_counts, impl_->sort_mode,
-                                      impl_->d_problems, impl_->offsets(), impl_->perm(), impl_->order(),
-                                      impl_->header(), stream);
+  const hipError_t status =
+      ggk_moe_prepare(impl_->variant, impl_->path, &impl_->layout, d_counts, impl_->sort_mode, impl_->d_problems,
+                      impl_->offsets(), impl_->perm(), impl_->order(), impl_->header(), stream);
   if (status != hipSuccess) return status;
-  int recorded = 0;
-  status = ggk_launch_grouped_device_done(impl_->variant, impl_->path, impl_->addressing, impl_->d_problems,
+  return impl_->buffer.tracked_launch(stream, true, [&](hipEvent_t done, int* recorded) {
+    return ggk_launch_grouped_device_done(impl_->variant, impl_->path, impl_->addressing, impl_->d_problems,
                                           impl_->offsets() + impl_->layout.experts + 1, impl_->order(),
                                           impl_->layout.experts, impl_->header(), impl_->d_state, impl_->grid_ctas,
-                                          impl_->buffer.last_launch, &recorded, stream);
-  if (status == hipSuccess) impl_->buffer.note_launch(recorded);
-  return status;
+                                          done, recorded, stream);
+  });
 }
 
 int MoeGroupedGemm::grid_ctas() const { return impl_ != nullptr ? impl_->grid_ctas : 0; }

@@ -140,9 +140,9 @@ hipError_t ggk_device_synchronize(void);
 
 /* Completion tracking of an executor's launches (no reference counterpart: the
  * reference frees its buffers with cudaFree, which waits for the whole device).
- * An executor has each launch's completion signal its event (ggk_launch_*_done;
- * recorded after it for a traced launch) and
- * waits for it before it rewrites or frees the buffers those launches read.  A
+ * An executor has a launch's completion signal its event (ggk_launch_*_done) or
+ * records it after the launch (the first on a stream, every 64th, traced ones)
+ * and waits for it before it rewrites or frees the buffers those launches read.  A
  * launch captured into a graph has no event (its replays run later, on streams
  * the executor never sees): the executor then waits for the whole device
  * instead.  Events are created with timing disabled. */
