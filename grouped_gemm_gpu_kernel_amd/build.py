@@ -14,6 +14,7 @@ Usage: python -m grouped_gemm_gpu_kernel_amd.build [--no-tests] [--no-oracle]
 """
 from __future__ import annotations
 
+import json
 import os
 import re
 import shutil
@@ -28,6 +29,7 @@ CSRC_DIR = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB_DIR = PKG / "lib"
 LIB_NAME = "libgrouped_gemm_amd.so"
+FORMS_NAME = "gg_kernel_forms.json"  # resources of every compiled kernel form, beside the objects
 ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 HIPCC = str(ROCM / "bin" / "hipcc")
 ARCH = "gfx950"
@@ -57,25 +59,23 @@ def _run(cmd: list[str], capture_stderr: bool = False) -> str:
     return proc.stderr if capture_stderr else proc.stdout
 
 
-def parse_resource_report(report: str) -> list[tuple[int, ...]]:
-    """Rows (kind, variant, path, vgprs, agprs, sgprs, scratch, waves, lds) for
-    the untraced grouped kernels and the single-problem kernels in the 32-bit
-    addressing form."""
-    rows, cur = [], {}
+def parse_kernel_forms(report: str) -> list[dict]:
+    """Every form of gg_grouped_kernel and gg_single_kernel in the compiler's
+    resource report: kind (0 grouped, 1 single), variant, path, traced, wide
+    (64-bit addressing) and its vgprs, agprs, sgprs, scratch, waves, lds."""
+    forms, cur = [], {}
 
     def flush():
         m = _KERNEL.search(cur.get("Function Name", ""))
         if not m:
             return
         kind = 0 if m.group(1) == "grouped" else 1
-        if kind == 0 and (m.group(4) != "0" or m.group(6) != "0"):
-            return  # traced (same code plus instrumentation) or 64-bit addressing form
-        if kind == 1 and m.group(4) != "0":
-            return  # 64-bit addressing form
-        rows.append((kind, int(m.group(2)), int(m.group(3)), int(cur.get("VGPRs", 0)),
-                     int(cur.get("AGPRs", 0)), int(cur.get("TotalSGPRs", 0)),
-                     int(cur.get("ScratchSize [bytes/lane]", 0)),
-                     int(cur.get("Occupancy [waves/SIMD]", 0)), int(cur.get("LDS Size [bytes/block]", 0))))
+        forms.append({
+            "kind": kind, "variant": int(m.group(2)), "path": int(m.group(3)),
+            "traced": int(m.group(4)) if kind == 0 else 0, "wide": int(m.group(6) if kind == 0 else m.group(4)),
+            "vgprs": int(cur.get("VGPRs", 0)), "agprs": int(cur.get("AGPRs", 0)),
+            "sgprs": int(cur.get("TotalSGPRs", 0)), "scratch": int(cur.get("ScratchSize [bytes/lane]", 0)),
+            "waves": int(cur.get("Occupancy [waves/SIMD]", 0)), "lds": int(cur.get("LDS Size [bytes/block]", 0))})
 
     for line in report.splitlines():
         m = _REMARK.search(line)
@@ -86,7 +86,15 @@ def parse_resource_report(report: str) -> list[tuple[int, ...]]:
             cur = {}
         cur[m.group(1)] = m.group(2)
     flush()
-    return rows
+    return forms
+
+
+def parse_resource_report(report: str) -> list[tuple[int, ...]]:
+    """Rows (kind, variant, path, vgprs, agprs, sgprs, scratch, waves, lds) for
+    the untraced grouped kernels and the single-problem kernels in the 32-bit
+    addressing form (a traced kernel is the same code plus instrumentation)."""
+    return [(f["kind"], f["variant"], f["path"], f["vgprs"], f["agprs"], f["sgprs"], f["scratch"], f["waves"], f["lds"])
+            for f in parse_kernel_forms(report) if not f["traced"] and not f["wide"]]
 
 
 def build_library(out_path: Path | None = None, defines: tuple[str, ...] = (), csrc: Path | None = None) -> Path:
@@ -126,6 +134,7 @@ def build_library(out_path: Path | None = None, defines: tuple[str, ...] = (), c
         raise RuntimeError(f"expected 24 kernel resource rows, parsed {len(rows)}")
     table = "".join("    {%d, %d, %d, %d, %d, %d, %d, %d, %d},\n" % r for r in sorted(rows))
     (build_dir / "gg_resources_table.inc").write_text(table)
+    (build_dir / FORMS_NAME).write_text(json.dumps(parse_kernel_forms(report)))
     res_o = build_dir / "gg_resources.o"
     _run([*CXX_FLAGS, f"-I{build_dir}", "-c", str(CSRC / "gg_resources.cpp"), "-o", str(res_o)])
 

@@ -195,7 +195,7 @@ template <int V> struct KernelShape<V, GGK_PATH_MFMA> {
   static constexpr int WAVE_M = kLarge && GG_WAVE_M < BM ? GG_WAVE_M : 64;                    // rows of D per wave
   static constexpr int THREADS = (BM / WAVE_M) * (BN / WAVE_N) * kWave;
   // Waves each SIMD must be able to hold (bounds the registers per lane).
-  static constexpr int WAVES_PER_EU = kLarge ? GG_TUNED_WAVES_PER_EU : 2;
+  static constexpr int waves_per_eu(bool) { return kLarge ? GG_TUNED_WAVES_PER_EU : 2; }
   // Stages load straight into LDS.  A 512-thread workgroup has a CU to
   // itself and takes three buffers (two stages in flight) when they fit in
   // LDS, else two; a 256-thread one takes two, so that two of its workgroups
@@ -227,8 +227,12 @@ template <int V> struct KernelShape<V, GGK_PATH_FMA> {
   static constexpr int TN = 1;
   // A 64 x 64 tile needs 128 registers and 32 KB of LDS: four workgroups a CU.
   // The larger tiles need more than a third of the registers (at three waves
-  // per SIMD they spill).
-  static constexpr int WAVES_PER_EU = VariantTile<V>::M * VariantTile<V>::N <= 64 * 64 ? 4 : 2;
+  // per SIMD they spill), and so does the 64-bit addressing form of every tile,
+  // which holds two stages in registers: bound to 128, the 64 x 64 tile's
+  // spilled 35 of them (100 bytes of scratch a lane).
+  static constexpr int waves_per_eu(bool wide) {
+    return !wide && VariantTile<V>::M * VariantTile<V>::N <= 64 * 64 ? 4 : 2;
+  }
   using G = Geometry<VariantTile<V>::M, VariantTile<V>::N, GG_STAGE_K, 2, 256>;
   static constexpr bool CLASSES = false;
 };

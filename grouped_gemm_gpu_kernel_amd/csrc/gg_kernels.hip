@@ -263,14 +263,14 @@ __device__ __forceinline__ void mark_tile_start(const PhaseStamps& stamps, int h
   stamps.mark(GGK_PHASE_START);
 }
 
-// At least KernelShape::WAVES_PER_EU waves per SIMD: 2 allows 256 VGPRs +
-// AGPRs per lane (a 512-thread workgroup, or two 256-thread ones), 1 allows 512.
-#define GG_KERNEL_ATTRS(V, PATH)                          \
+// At least this many waves per SIMD (KernelShape): 4 allows 128 VGPRs + AGPRs
+// per lane, 3 allows 168, 2 (a 512-thread workgroup, or two 256-thread ones) 256.
+#define GG_KERNEL_ATTRS(V, PATH, WIDE)                    \
   __launch_bounds__((KernelShape<V, PATH>::G::THREADS)) \
-      __attribute__((amdgpu_waves_per_eu(KernelShape<V, PATH>::WAVES_PER_EU)))
+      __attribute__((amdgpu_waves_per_eu(KernelShape<V, PATH>::waves_per_eu(WIDE))))
 
 template <int V, int PATH, bool TRACED, bool WIDE>
-__global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
+__global__ GG_KERNEL_ATTRS(V, PATH, WIDE) void gg_grouped_kernel(GroupedArgs args) {
   using S = KernelShape<V, PATH>;
   using G = typename S::G;
   __shared__ StageRing<KernelLds<S>::HALVES> lds;
@@ -461,7 +461,7 @@ __global__ GG_KERNEL_ATTRS(V, PATH) void gg_grouped_kernel(GroupedArgs args) {
 }
 
 template <int V, int PATH, bool WIDE>
-__global__ GG_KERNEL_ATTRS(V, PATH) void gg_single_kernel(gg_device_problem_desc p) {
+__global__ GG_KERNEL_ATTRS(V, PATH, WIDE) void gg_single_kernel(gg_device_problem_desc p) {
   using S = KernelShape<V, PATH>;
   using G = typename S::G;
   __shared__ StageRing<KernelLds<S>::HALVES> lds;
