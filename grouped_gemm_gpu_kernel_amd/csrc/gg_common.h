@@ -225,13 +225,12 @@ template <int V> struct KernelShape<V, GGK_PATH_MFMA> {
 template <int V> struct KernelShape<V, GGK_PATH_FMA> {
   static constexpr int TM = 1;
   static constexpr int TN = 1;
-  // A 64 x 64 tile needs 128 registers and 32 KB of LDS: four workgroups a CU.
-  // The larger tiles need more than a third of the registers (at three waves
-  // per SIMD they spill), and so does the 64-bit addressing form of every tile,
-  // which holds two stages in registers: bound to 128, the 64 x 64 tile's
-  // spilled 35 of them (100 bytes of scratch a lane).
+  // Workgroups a CU holds, which the registers have to allow: four of a 64 x 64
+  // tile (32 KB of LDS each), three of the larger ones (48 KB).  The 64-bit
+  // addressing form holds two stages in registers and has a bound of its own:
+  // at 128 registers the 64 x 64 tile's spilled 35 of them.
   static constexpr int waves_per_eu(bool wide) {
-    return !wide && VariantTile<V>::M * VariantTile<V>::N <= 64 * 64 ? 4 : 2;
+    return wide ? 2 : VariantTile<V>::M * VariantTile<V>::N <= 64 * 64 ? 4 : 3;
   }
   using G = Geometry<VariantTile<V>::M, VariantTile<V>::N, GG_STAGE_K, 2, 256>;
   static constexpr bool CLASSES = false;

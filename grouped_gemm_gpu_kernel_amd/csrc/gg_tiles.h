@@ -242,15 +242,19 @@ __device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& 
   if constexpr (!std::is_same_v<Stamps, NoStamps>) phase_barrier();
 }
 
-// The FMA path's k-loop with stage loads straight into LDS: compute(stage,
-// first k) once per stage.  A stage's buffer is asked for stage t + 2 when
-// every wave has multiplied stage t, so no load waits in registers, and one
-// copy of the multiplying code serves every stage.  Staged through a ring of
-// three register sets the code came in five copies (40 KB) and a CU held two
-// workgroups of 64 x 64 tiles; it holds four with 32 KB of LDS each.  256 problems of
-// 16 to 256 in each dimension (893 tiles): 31.2 -> 29.3 us, with FmaTile's
-// vector epilogue 26.0.  A launch like that is bound by each tile's own chain:
-// a 64 x 64 tile 256 deep takes 6.8 us of FMAs, all tiles together 5.9 us of the chip.
+// The FMA path's k-loop with stage loads straight into LDS:
+// compute(stage, first k, issue) once per stage, which calls issue(l) for l = 0
+// .. LOADS - 1 somewhere in it.  Stages t and t + 1 share two buffers: while
+// stage t is multiplied, issue asks for the loads of stage t + 1, into the
+// buffer that every wave has left since the barrier before (the first two
+// stages are asked for ahead of the loop).  One wait and one barrier a stage.
+// No load waits in registers, and one copy of the multiplying code serves every
+// stage: staged through a ring of three register sets it came in five copies
+// (40 KB).  256 problems of 16 to 256 in each dimension (893 tiles): 31.2 ->
+// 29.3 us, with FmaTile's vector epilogue 26.0, with every tile fixed 21.2, with
+// the unrolled slices 20.8.  A launch like that is bound by each tile's own
+// chain: a 64 x 64 tile 256 deep takes 6.8 us of FMAs, all tiles together 5.9 us
+// of the chip.
 template <class G, class Compute, class OnStart, class Stamps>
 __device__ __forceinline__ void run_k_loop_fma(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
                                                Compute&& compute, OnStart&& on_start, const Stamps& stamps) {
@@ -267,23 +271,29 @@ __device__ __forceinline__ void run_k_loop_fma(const gg_device_problem_desc& p, 
   loader.issue(0, lds);
   if (nk > 1) loader.issue(1, lds + G::STAGE);
   const bool extra = __builtin_amdgcn_readfirstlane(on_start() ? 1 : 0) != 0;
+  // In flight behind the loads of stage 0: those of stage 1 and the request.
+  if (nk == 1) {
+    if (extra) wait_vmcnt<1>(); else wait_vmcnt<0>();
+  } else {
+    if (extra) wait_vmcnt<LOADS + 1>(); else wait_vmcnt<LOADS>();
+  }
+  stamps.mark(GGK_PHASE_FIRST_STAGE);
+  if (loader.last_stage == 0) loader.fix_last_stage(0, lds);
+  stage_barrier();
+  stamps.mark(GGK_PHASE_K_LOOP);
 #pragma unroll 1
   for (int t = 0; t < nk; ++t) {
     uint16_t* const stage = lds + (t & 1) * G::STAGE;
-    // In flight behind the loads of stage t: those of stage t + 1 and, at the start, the request.
-    if (t + 1 == nk) {
+    uint16_t* const next = lds + ((t + 1) & 1) * G::STAGE;
+    const bool ask = t > 0 && t + 1 < nk;
+    compute(stage, t * G::BK, [&](int l) {
+      if (ask) loader.issue_load(t + 1, next, l);
+    });
+    if (t + 1 < nk) {
+      // The loads of stage t + 1; the request made at the start may stay in flight once.
       if (t == 0 && extra) wait_vmcnt<1>(); else wait_vmcnt<0>();
-    } else {
-      if (t == 0 && extra) wait_vmcnt<LOADS + 1>(); else wait_vmcnt<LOADS>();
-    }
-    if (t == 0) stamps.mark(GGK_PHASE_FIRST_STAGE);
-    if (t == loader.last_stage) loader.fix_last_stage(t, stage);
-    stage_barrier();
-    if (t == 0) stamps.mark(GGK_PHASE_K_LOOP);
-    compute(stage, t * G::BK);
-    if (t + 2 < nk) {
+      if (t + 1 == loader.last_stage) loader.fix_last_stage(t + 1, next);
       stage_barrier();
-      loader.issue(t + 2, stage);
     }
   }
 }
@@ -594,9 +604,15 @@ struct MfmaTile {
 // tm*RM .. tm*RM+RM-1 and columns tn*RN .. tn*RN+RN-1 of the macro-tile, with
 // RM = BM/16, RN = BN/16 float32 accumulators.  Per 8-deep k slice a thread
 // reads one 16-byte piece of each of its A rows and one RN-wide piece of each
-// B row from LDS (while the slice before is multiplied), then issues RM*RN*8
-// fused multiply-adds in ascending k.
+// B row from LDS, then issues RM*RN*8 fused multiply-adds in ascending k.
 // Used when MFMA is not requested (use_tensor_cores = false).
+//
+// The slices of a stage are unrolled and left to the compiler to schedule.
+// Reading each slice ahead of the one being multiplied needs another RM*4 +
+// RN*4 registers: the larger tiles then hold two workgroups a CU instead of
+// three, and every tile pays in issue slots.  37 problems of 300 to 1400 rows and
+// columns, K 256 to 512: 64x64x16 348 -> 333 us, 128x64x32 374 -> 350, 64x128x32
+// 358 -> 340; 300 problems of 16 to 400: 41.3 -> 40.4, 65 -> 62, 64.8 -> 54.8.
 // ---------------------------------------------------------------------------
 template <class G>
 struct FmaTile {
@@ -605,49 +621,51 @@ struct FmaTile {
   static_assert(RN == 4 || RN == 8, "column block must be one or two LDS chunks");
   static_assert(G::THREADS == 256, "16 x 16 thread grid");
 
-  // The operands of an 8-deep slice of a stage: RM rows of A, 8 k-rows of B.
-  using brow_t = std::conditional_t<RN == 4, half4_t, half8_t>;
-  struct Slice {
-    half8_t a[RM];
-    brow_t b[8];
-  };
-  __device__ __forceinline__ static void load_slice(const uint16_t* stage, int k8, int tm, int tn, Slice& s) {
+  // One accumulator tile of 4 x 4 leaves registers for C beside the k-loop's.
+  static constexpr bool SMALL = RM * RN <= 16;
+  static constexpr int SLICES = G::BK / 8;
+  static constexpr int LOADS = DmaLoader<G>::LOADS;
+  static_assert(LOADS <= SLICES, "a stage's loads go out one a slice");
+
+  // Multiplies a stage whose first krem values of k lie inside the problem.
+  // issue(l) asks for load l of the next stage: one a slice behind its operand
+  // reads in the 4 x 4 form, where a lone workgroup has nothing else to hide
+  // them behind (64 problems 1024 to 4096 deep: 193 -> 187 us), else all ahead of
+  // the slices (the larger tiles lose up to 4% with the loads spread out).
+  template <class Issue>
+  __device__ __forceinline__ static void compute_stage(const uint16_t* stage, int krem, int tm, int tn,
+                                                       float (&acc)[RM][RN], Issue&& issue) {
+    using brow_t = std::conditional_t<RN == 4, half4_t, half8_t>;
+    if constexpr (!SMALL) issue_all(issue);
 #pragma unroll
-    for (int i = 0; i < RM; ++i) s.a[i] = *reinterpret_cast<const half8_t*>(stage + G::a_piece(tm * RM + i, k8));
+    for (int k8 = 0; k8 < SLICES; ++k8) {
+      if (k8 * 8 >= krem) break;  // loads follow full stages only
+      half8_t av[RM];
+      brow_t bv[8];
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      s.b[kk] = *reinterpret_cast<const brow_t*>(stage + G::A_STAGE + G::b_chunk(k8 * 8 + kk, tn * RN));
-    }
-  }
-  __device__ __forceinline__ static void multiply_slice(const Slice& s, float (&acc)[RM][RN]) {
+      for (int i = 0; i < RM; ++i) av[i] = *reinterpret_cast<const half8_t*>(stage + G::a_piece(tm * RM + i, k8));
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
+      for (int kk = 0; kk < 8; ++kk) {
+        bv[kk] = *reinterpret_cast<const brow_t*>(stage + G::A_STAGE + G::b_chunk(k8 * 8 + kk, tn * RN));
+      }
+      if constexpr (SMALL) {
+        if (k8 < LOADS) issue(k8);
+      }
 #pragma unroll
-      for (int i = 0; i < RM; ++i) {
-        const float a = (float)s.a[i][kk];
+      for (int kk = 0; kk < 8; ++kk) {
 #pragma unroll
-        for (int j = 0; j < RN; ++j) acc[i][j] = __builtin_fmaf(a, (float)s.b[kk][j], acc[i][j]);
+        for (int i = 0; i < RM; ++i) {
+          const float a = (float)av[i][kk];
+#pragma unroll
+          for (int j = 0; j < RN; ++j) acc[i][j] = __builtin_fmaf(a, (float)bv[kk][j], acc[i][j]);
+        }
       }
     }
   }
-  __device__ __forceinline__ static void compute_stage(const uint16_t* stage, int krem, int tm, int tn,
-                                                       float (&acc)[RM][RN]) {
-    const int slices = krem >= G::BK ? G::BK / 8 : (krem + 7) / 8;
-    // The next slice is read while this one is multiplied (past the last: one that is not used).
-    Slice even, odd;
-    load_slice(stage, 0, tm, tn, even);
-#pragma unroll 1
-    for (int k8 = 0; k8 < slices; k8 += 2) {
-      load_slice(stage, k8 + 1, tm, tn, odd);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply_slice(even, acc);
-      __builtin_amdgcn_sched_barrier(0);
-      if (k8 + 1 == slices) break;
-      load_slice(stage, (k8 + 2) % (G::BK / 8), tm, tn, even);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply_slice(odd, acc);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+  template <class Issue>
+  __device__ __forceinline__ static void issue_all(Issue&& issue) {
+#pragma unroll
+    for (int l = 0; l < LOADS; ++l) issue(l);
   }
 
   // Computes the work tile at (m0, n0); on_start and after_k_loop as in
@@ -668,42 +686,50 @@ struct FmaTile {
       for (int j = 0; j < RN; ++j) acc[i][j] = 0.0f;
 
     // The thread's part of C, as 16-byte vectors through a buffer resource from
-    // the wave's first row (vectors past N read as zero), asked for before the
-    // k-loop's loads.  Read and written as dwords after the k-loop: 29.3 us
-    // where this takes 26.0 (256 problems of 16 to 256 in each dimension).
+    // the wave's first row (vectors past N read as zero).  The 4 x 4 form asks
+    // for it before the k-loop's loads (read and written as dwords after the
+    // k-loop: 29.3 us where this takes 26.0, 256 problems of 16 to 256 in each
+    // dimension), the others, which have no registers left for it beside three
+    // waves per SIMD, when the k-loop ends, ahead of the hand-over.
     const bool use_c = p.c != nullptr && p.beta != 0.0f;
     const int r0 = __builtin_amdgcn_readfirstlane(m0 + (tid / kWave) * 4 * RM);
-    const int row_lane = ((tid & (kWave - 1)) >> 4) * RM;
-    floatx4_t early[RM][RN / 4];
+    floatx4_t cv[RM][RN / 4];
+    auto request_c = [&](int t) {
 #pragma unroll
-    for (int i = 0; i < RM; ++i)
+      for (int i = 0; i < RM; ++i)
 #pragma unroll
-      for (int v = 0; v < RN / 4; ++v) early[i][v] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    if (!WIDE && use_c && active) {
+        for (int v = 0; v < RN / 4; ++v) cv[i][v] = floatx4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      if (WIDE || !use_c || !active) return;
       const __amdgpu_buffer_rsrc_t crs =
           buffer_rsrc(p.c + ((int64_t)r0 * p.ldc + n0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldc + (p.n - n0)));
 #pragma unroll
       for (int i = 0; i < RM; ++i)
 #pragma unroll
         for (int v = 0; v < RN / 4; ++v) {
-          const int col = tn * RN + 4 * v;
-          const uint32_t off = n0 + col < p.n ? 4u * ((uint32_t)(row_lane + i) * (uint32_t)p.ldc + (uint32_t)col)
+          const int row = ((t & (kWave - 1)) >> 4) * RM + i, col = (t & 15) * RN + 4 * v;
+          const uint32_t off = n0 + col < p.n ? 4u * ((uint32_t)row * (uint32_t)p.ldc + (uint32_t)col)
                                               : DmaLoader<G>::kOutOfRange;
-          early[i][v] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(crs, (int)off, 0, 0));
+          cv[i][v] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(crs, (int)off, 0, 0));
         }
-    }
+    };
+    if constexpr (SMALL) request_c(tid);
 
     if constexpr (WIDE) {
       int kt = 0;
       run_k_loop<G>(p, m0, n0, lds, [&](const uint16_t* stage) {
-        if (active) compute_stage(stage, p.k - kt * G::BK, tm, tn, acc);
+        if (active) compute_stage(stage, p.k - kt * G::BK, tm, tn, acc, [](int) {});
         ++kt;
       }, on_start, stamps);
     } else {
-      run_k_loop_fma<G>(p, m0, n0, lds, [&](const uint16_t* stage, int k0) {
-        if (active) compute_stage(stage, p.k - k0, tm, tn, acc);
+      run_k_loop_fma<G>(p, m0, n0, lds, [&](const uint16_t* stage, int k0, auto&& issue) {
+        if (active) {
+          compute_stage(stage, p.k - k0, tm, tn, acc, issue);
+        } else {
+          issue_all(issue);
+        }
       }, on_start, stamps);
     }
+    if constexpr (!SMALL) request_c(opaque_tid());
     after_k_loop();
 
     if (!active) {
@@ -717,34 +743,35 @@ struct FmaTile {
       for (int i = 0; i < RM; ++i) {
         const int row = m0 + tm * RM + i;
         if (row >= p.m) continue;
-        float cv[RN];
+        float ce[RN];
 #pragma unroll
         for (int j = 0; j < RN; ++j) {
           const int col = n0 + tn * RN + j;
-          cv[j] = (use_c && col < p.n) ? cptr[(int64_t)row * p.ldc + col] : 0.0f;
+          ce[j] = (use_c && col < p.n) ? cptr[(int64_t)row * p.ldc + col] : 0.0f;
         }
 #pragma unroll
         for (int j = 0; j < RN; ++j) {
           const int col = n0 + tn * RN + j;
-          if (col < p.n) dptr[(int64_t)row * p.ldd + col] = epilogue_value(acc[i][j], cv[j], p.alpha, use_c ? p.beta : 0.0f);
+          if (col < p.n) dptr[(int64_t)row * p.ldd + col] = epilogue_value(acc[i][j], ce[j], p.alpha, use_c ? p.beta : 0.0f);
         }
       }
     } else {
+      const int t = opaque_tid();  // its parts are not held through the k-loop
       const __amdgpu_buffer_rsrc_t drs =
           buffer_rsrc(p.d + ((int64_t)r0 * p.ldd + n0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldd + (p.n - n0)));
 #pragma unroll
       for (int i = 0; i < RM; ++i) {
-        const int row = row_lane + i;
+        const int row = ((t & (kWave - 1)) >> 4) * RM + i;
         if (r0 + row >= p.m) continue;
 #pragma unroll
         for (int v = 0; v < RN / 4; ++v) {
-          const int col = tn * RN + 4 * v;
+          const int col = (t & 15) * RN + 4 * v;
           const int ncol = p.n - (n0 + col);
           const uint32_t off = 4u * ((uint32_t)row * (uint32_t)p.ldd + (uint32_t)col);
           floatx4_t out;
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            out[e] = epilogue_value(acc[i][4 * v + e], early[i][v][e], p.alpha, use_c ? p.beta : 0.0f);
+            out[e] = epilogue_value(acc[i][4 * v + e], cv[i][v][e], p.alpha, use_c ? p.beta : 0.0f);
           }
           if (ncol >= 4) {
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) int, out), drs,

@@ -13,7 +13,6 @@ MFMA, FMA = 1, 0
 
 # Bytes of scratch a lane that a form may have.
 KNOWN = {(0, v, MFMA, traced, 0): 32 if traced else 8 for v in LARGE for traced in (0, 1)}
-KNOWN.update({(0, v, FMA, 1, 0): 20 for v in (0, 5)})  # 64 x 64 tiles
 
 
 def _forms():
@@ -42,3 +41,10 @@ def test_no_selectable_form_spills():
         if f["scratch"] > KNOWN.get(_key(f), 0):
             spills[_key(f)] = f["scratch"]
     assert not spills, f"(kind, variant, path, traced, wide): bytes of scratch a lane {spills}"
+
+
+def test_fma_registers_allow_the_workgroups_that_lds_holds():
+    """160 KB of LDS hold four 64 x 64 tiles or three larger ones; a workgroup is one wave per SIMD."""
+    for f in _forms():
+        if f["path"] == FMA and not f["wide"]:
+            assert f["waves"] >= (4 if f["variant"] in (0, 5) else 3), f
