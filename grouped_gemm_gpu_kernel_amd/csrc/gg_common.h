@@ -236,6 +236,19 @@ template <int V> struct KernelShape<V, GGK_PATH_FMA> {
   static constexpr bool CLASSES = false;
 };
 
+// The lane, and the thread index of a wave of the workgroup, counted where they
+// are used.  The empty asm makes the compiler assume that the lane changes at
+// every call, so that neither it nor what is derived from it is held in
+// registers for the whole persistent kernel; the wave's index is a scalar.  With
+// threadIdx.x itself behind the asm its register stayed taken, and the 256 x 256
+// kernels, which use all 256, spilled it.
+__device__ __forceinline__ int opaque_lane() {
+  int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+__device__ __forceinline__ int opaque_tid(int wave) { return wave * kWave + opaque_lane(); }
+
 // Per-work-tile phase stamps of a traced launch: 8 int64 per work-tile index
 // (GGK_PHASE_* in grouped_gemm_amd_kernels.h).  Core-clock stamps are
 // s_memtime; one wave's record stands for the workgroup except the epilogue
@@ -248,15 +261,15 @@ struct NoStamps {
 };
 struct PhaseStamps {
   long long* slot;  // this work tile's 8 entries, or null
+  int wave;         // uniform
   __device__ __forceinline__ void mark(int i) const {
-    if (slot != nullptr && __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) == 0) {
+    if (slot != nullptr && wave == 0) {
       slot[i] = static_cast<long long>(__builtin_amdgcn_s_memtime());
     }
   }
   // Every wave (lane 0): mark i of the k-loop step that is stamped (GGK_PHASE_STEP).
   __device__ __forceinline__ void step_mark(int i) const {
     if (slot != nullptr && (threadIdx.x & (kWave - 1)) == 0) {
-      const int wave = threadIdx.x / kWave;
       slot[GGK_PHASE_STEP + GGK_PHASE_STEP_MARKS * wave + i] = static_cast<long long>(__builtin_amdgcn_s_memtime());
     }
   }
@@ -268,15 +281,6 @@ struct PhaseStamps {
     }
   }
 };
-
-// threadIdx.x behind an empty asm: the compiler must assume it changes at
-// every call, so values derived from it are recomputed where they are used
-// instead of being held in registers for the whole persistent kernel.
-__device__ __forceinline__ int opaque_tid() {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
-}
 
 // Global-memory views.  Descriptor pointers arrive as generic pointers; the
 // kernels only ever point them at device memory, so they are read and written
@@ -429,11 +433,12 @@ struct StageLoader {
   static constexpr int BPR = G::BN / 8;  // B pieces per k-row
 
   const gg_device_problem_desc& p;
+  int wave;  // uniform
   int tid;
   int m0, n0;
 
-  __device__ __forceinline__ StageLoader(const gg_device_problem_desc& prob, int m0_, int n0_)
-      : p(prob), tid(opaque_tid()), m0(m0_), n0(n0_) {}
+  __device__ __forceinline__ StageLoader(const gg_device_problem_desc& prob, int m0_, int n0_, int wave_)
+      : p(prob), wave(wave_), tid(opaque_tid(wave_)), m0(m0_), n0(n0_) {}
 
   __device__ __forceinline__ EdgePlace a_edge(int i, int kt) const {
     const int v = tid + i * T;
@@ -452,7 +457,7 @@ struct StageLoader {
   }
 
   __device__ __forceinline__ void store(const RawStage<G>& r, int kt, uint16_t* lds, int s) const {
-    const int t = opaque_tid();
+    const int t = opaque_tid(wave);
     uint16_t* as = lds + s * G::STAGE;
     uint16_t* bs = as + G::A_STAGE;
 #pragma unroll
@@ -553,11 +558,9 @@ struct DmaLoader {
   bool a_fix, b_fix;  // whether the matrices' last values must be put back (see the constructor)
   uint32_t a_last, b_last;
 
-  __device__ __forceinline__ DmaLoader(const gg_device_problem_desc& p, int m0_, int n0_)
-      : m(p.m), n(p.n), k(p.k), ldb(p.ldb), m0(m0_), n0(n0_) {
-    const int tid = opaque_tid();
-    const int lane = tid & (kWave - 1);
-    wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  __device__ __forceinline__ DmaLoader(const gg_device_problem_desc& p, int m0_, int n0_, int wave_)
+      : m(p.m), n(p.n), k(p.k), ldb(p.ldb), wave(wave_), m0(m0_), n0(n0_) {
+    const int lane = opaque_lane();
     const uint16_t* A = static_cast<const uint16_t*>(p.a);
     const uint16_t* B = static_cast<const uint16_t*>(p.b);
     a_tile = A + (int64_t)m0 * p.lda;
@@ -633,7 +636,7 @@ struct DmaLoader {
     int a_col8 = this->a_col8, b_col8 = this->b_col8, m0 = this->m0, n0 = this->n0;
     asm volatile("" : "+s"(k), "+s"(m), "+s"(n), "+s"(m0), "+s"(n0), "+s"(kt));
     asm volatile("" : "+v"(a_row), "+v"(b_row), "+v"(a_col8), "+v"(b_col8));
-    const int lane = opaque_tid() & (kWave - 1);
+    const int lane = opaque_lane();
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       u32x4_t* slot = reinterpret_cast<u32x4_t*>(stage + (i * WAVES + wave) * (kWave * 8) + 8 * lane);

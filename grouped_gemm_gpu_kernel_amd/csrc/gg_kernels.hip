@@ -252,7 +252,7 @@ __device__ __forceinline__ void work_tile_position(int local, int wtm, int wtn, 
 template <class G>
 __device__ __forceinline__ void mark_tile_start(const PhaseStamps& stamps, int half, const gg_device_problem_desc& p,
                                                 int m0, int n0) {
-  if (stamps.slot != nullptr && __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) == 0) {
+  if (stamps.slot != nullptr && stamps.wave == 0) {
     const long long rows = p.m - m0 < G::BM ? p.m - m0 : G::BM;
     const long long cols = p.n - n0 < G::BN ? p.n - n0 : G::BN;
     const long long stages = (p.k + G::BK - 1) / G::BK;
@@ -279,7 +279,8 @@ __global__ GG_KERNEL_ATTRS(V, PATH, WIDE) void gg_grouped_kernel(GroupedArgs arg
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  const bool wave0 = __builtin_amdgcn_readfirstlane(tid / kWave) == 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const bool wave0 = wave == 0;
   long long clock_start = 0;
   long long clock_end = 0;
   if (TRACED) {
@@ -371,7 +372,8 @@ __global__ GG_KERNEL_ATTRS(V, PATH, WIDE) void gg_grouped_kernel(GroupedArgs arg
     // Phase stamps of this work tile (traced launches with a phase buffer only).
     static_assert(G::THREADS <= kWave * GGK_PHASE_STEP_WAVES, "one step-stamp row per wave");
     PhaseStamps stamps{TRACED && args.tile_phases != nullptr ? args.tile_phases + (long long)GGK_PHASE_COUNT * t
-                                                             : nullptr};
+                                                             : nullptr,
+                       wave};
     auto after_k_loop = [&]() {
       stamps.mark(GGK_PHASE_K_END);
       if (!asked) request();
@@ -429,9 +431,9 @@ __global__ GG_KERNEL_ATTRS(V, PATH, WIDE) void gg_grouped_kernel(GroupedArgs arg
         if (split != 0 && n0 + G::BN / 2 < p.n) q.n = n0 + G::BN / 2;
         if constexpr (TRACED) {
           mark_tile_start<G>(stamps, half, q, m0, n0);
-          run_work_tile<S, PATH, WIDE>(q, m0, n0, lds, request, after_k_loop, stamps);
+          run_work_tile<S, PATH, WIDE>(q, m0, n0, lds, wave, request, after_k_loop, stamps);
         } else if (!kSplits || n0 < p.n) {  // else: an empty second half
-          run_work_tile<S, PATH, WIDE>(q, m0, n0, lds, request, after_k_loop);
+          run_work_tile<S, PATH, WIDE>(q, m0, n0, lds, wave, request, after_k_loop);
         }
       }
     }
@@ -471,7 +473,8 @@ __global__ GG_KERNEL_ATTRS(V, PATH, WIDE) void gg_single_kernel(gg_device_proble
   if (wtn <= 0 || t >= wtm * wtn) return;
   const int wm = t / wtn;
   const int wn = t - wm * wtn;
-  run_work_tile<S, PATH, WIDE>(p, wm * G::BM, wn * G::BN, lds, [] { return false; }, [] {});
+  run_work_tile<S, PATH, WIDE>(p, wm * G::BM, wn * G::BN, lds,
+                               __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), [] { return false; }, [] {});
 }
 
 // ---------------------------------------------------------------------------

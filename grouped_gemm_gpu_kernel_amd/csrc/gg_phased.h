@@ -76,10 +76,9 @@ struct PhasedLoader {
   int last_stage;
   bool fix_a, fix_b;  // the units of the last stage need repair (see repair_a, repair_b)
 
-  __device__ __forceinline__ PhasedLoader(const gg_device_problem_desc& p, int m0_, int n0_)
-      : m(p.m), n(p.n), k(p.k), ldb(p.ldb), m0(m0_), n0(n0_) {
-    const int tid = opaque_tid();
-    wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  __device__ __forceinline__ PhasedLoader(const gg_device_problem_desc& p, int m0_, int n0_, int wave_)
+      : m(p.m), n(p.n), k(p.k), ldb(p.ldb), wave(wave_), m0(m0_), n0(n0_) {
+    const int tid = opaque_tid(wave);
     a_tile = static_cast<const uint16_t*>(p.a) + (int64_t)m0 * p.lda;
     a_n = DmaLoader<G>::records(2 * ((int64_t)(p.m - 1 - m0) * p.lda + p.k));
     b_tile = static_cast<const uint16_t*>(p.b) + n0;
@@ -121,7 +120,7 @@ struct PhasedLoader {
   // landed: values at k >= K become zero, and a matrix's last value is put
   // back where its straddling dword read as zero.
   __device__ __forceinline__ void repair_a(const gg_device_problem_desc& p, int half, uint16_t* unit) const {
-    const int tid = opaque_tid();
+    const int tid = opaque_tid(wave);
     const int a_row = tid / 8;
     const int col = last_stage * G::BK + 8 * ((tid & 7) ^ G::a_swizzle(a_row));
     const uint32_t last =
@@ -137,7 +136,7 @@ struct PhasedLoader {
     wait_lgkmcnt<0>();  // written before the barrier that follows
   }
   __device__ __forceinline__ void repair_b(const gg_device_problem_desc& p, int half, uint16_t* unit) const {
-    const int tid = opaque_tid();
+    const int tid = opaque_tid(wave);
     const int b_row = tid / 32;
     const int col = n0 + 8 * ((tid & 31) ^ (G::b_swizzle(b_row) >> 1));
     const bool odd = (n & 1) != 0 && n0 + G::BN >= n;
@@ -156,12 +155,12 @@ struct PhasedLoader {
   }
 };
 
-// Runs the k-loop of the full work tile at (m0, n0) for the wave at block row
+// Runs the k-loop of the full work tile at (m0, n0) for wave `wave`, at block row
 // wm (128 rows) and block column wn (64 columns); on_start as in the other
 // k-loops.
 template <class G, class OnStart, class Stamps>
-__device__ __forceinline__ void run_k_loop_phased(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds, int wm,
-                                                  int wn, floatx4_t (&acc)[8][4], OnStart&& on_start,
+__device__ __forceinline__ void run_k_loop_phased(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds, int wave,
+                                                  int wm, int wn, floatx4_t (&acc)[8][4], OnStart&& on_start,
                                                   const Stamps& stamps) {
   using L = PhasedLoader<G>;
   const int nk = (p.k + G::BK - 1) / G::BK;
@@ -169,11 +168,11 @@ __device__ __forceinline__ void run_k_loop_phased(const gg_device_problem_desc& 
     on_start();
     return;
   }
-  const L loader(p, m0, n0);
+  const L loader(p, m0, n0, wave);
 
   half8_t a[2][4][2];  // [A half][16-row block][32-deep k-step]
   half8_t b[2][4];     // [B half, one k-step][16-column block]
-  const int lane = opaque_tid() & (kWave - 1);
+  const int lane = opaque_lane();
   const int g = lane >> 4, j = lane & 15;
   // LDS byte address of the lane's fragment in the first units: block 0, k-step 0
   // (operand layouts as in MfmaTile).

@@ -36,14 +36,14 @@ namespace gg {
 // is addressed statically.
 template <class G, class Compute, class OnStart, class Stamps>
 __device__ __forceinline__ void run_k_loop(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
-                                           Compute&& compute, OnStart&& on_start, const Stamps& stamps) {
+                                           int wave, Compute&& compute, OnStart&& on_start, const Stamps& stamps) {
   constexpr int D = G::DEPTH;
   const int nk = (p.k + G::BK - 1) / G::BK;
   if (nk <= 0) {
     on_start();
     return;
   }
-  const StageLoader<G> loader(p, m0, n0);
+  const StageLoader<G> loader(p, m0, n0, wave);
   RawStage<G> ring[D];
 #pragma unroll
   for (int s = 0; s < D - 1; ++s) loader.issue(s, ring[s]);
@@ -94,8 +94,8 @@ __device__ __forceinline__ void run_k_loop(const gg_device_problem_desc& p, int 
 // on_start runs after the first barrier: the request it makes is then the
 // youngest operation in flight, and the first stage's wait lets it stay there.
 template <class G, int WM, class OnStart, class Stamps>
-__device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds, int wm,
-                                                  int wn, floatx4_t (&acc)[WM / 16][4], OnStart&& on_start,
+__device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds, int wave,
+                                                  int wm, int wn, floatx4_t (&acc)[WM / 16][4], OnStart&& on_start,
                                                   const Stamps& stamps) {
   using L = DmaLoader<G>;
   constexpr int NBUF = G::BUFFERS;
@@ -108,7 +108,7 @@ __device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& 
     on_start();
     return;
   }
-  const L loader(p, m0, n0);
+  const L loader(p, m0, n0, wave);
   const bool deep = nk >= NBUF;  // every buffer gets a stage
 #pragma unroll
   for (int s = 0; s < NBUF - 1; ++s) {
@@ -129,7 +129,7 @@ __device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& 
 
   half8_t a[2][FM];  // [k-half][16-row block]
   half8_t b[2][4];   // [k-half][16-column block]
-  const int lane = opaque_tid() & (kWave - 1);
+  const int lane = opaque_lane();
   const int g = lane >> 4, j = lane & 15;
   // LDS byte address of the lane's fragments of block 0, k-half 0 (operand layouts as in MfmaTile).
   const uint32_t a_lane = lds_address(lds) + 2u * (uint32_t)G::a_piece(wm * WM + j, g);
@@ -257,7 +257,7 @@ __device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& 
 // of the chip.
 template <class G, class Compute, class OnStart, class Stamps>
 __device__ __forceinline__ void run_k_loop_fma(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
-                                               Compute&& compute, OnStart&& on_start, const Stamps& stamps) {
+                                               int wave, Compute&& compute, OnStart&& on_start, const Stamps& stamps) {
   using L = DmaLoader<G>;
   constexpr int NBUF = G::BUFFERS;
   constexpr int LOADS = L::LOADS;
@@ -267,7 +267,7 @@ __device__ __forceinline__ void run_k_loop_fma(const gg_device_problem_desc& p, 
     on_start();
     return;
   }
-  const L loader(p, m0, n0);
+  const L loader(p, m0, n0, wave);
   loader.issue(0, lds);
   if (nk > 1) loader.issue(1, lds + G::STAGE);
   const bool extra = __builtin_amdgcn_readfirstlane(on_start() ? 1 : 0) != 0;
@@ -356,7 +356,7 @@ struct MfmaTile {
                                                        floatx4_t (&acc)[FM][FN]) {
     const uint16_t* as = stage;
     const uint16_t* bs = stage + G::A_STAGE;
-    lane = opaque_tid() & (kWave - 1);
+    lane = opaque_lane();
     const int g = lane >> 4;
     const int j = lane & 15;
     // Operand fragments of k-step s (32 deep) of the stage.
@@ -392,15 +392,13 @@ struct MfmaTile {
     }
   }
 
-  // Computes the work tile at (m0, n0); on_start as in the k-loops, and
+  // Computes the work tile at (m0, n0) as wave `wave`; on_start as in the k-loops, and
   // after_k_loop() once by every thread when the k-loop is over (no LDS read
   // of this tile follows it: the epilogue works from registers).
   template <bool WIDE, class OnStart, class AfterKLoop, class Stamps>
   __device__ __forceinline__ static void run(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
-                                             OnStart&& on_start, AfterKLoop&& after_k_loop, const Stamps& stamps) {
-    const int tid = opaque_tid();
-    const int lane = tid & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+                                             int wave, OnStart&& on_start, AfterKLoop&& after_k_loop, const Stamps& stamps) {
+    const int lane = opaque_lane();
     const int wm = wave / WAVES_N;
     const int wn = wave % WAVES_N;
     // A wave whose block starts past the problem's edge has nothing to
@@ -424,11 +422,11 @@ struct MfmaTile {
       if (live) compute_stage(stage, lane, wm, wn, acc);
     };
     if constexpr (WIDE) {
-      run_k_loop<G>(p, m0, n0, lds, compute, on_start, stamps);
+      run_k_loop<G>(p, m0, n0, lds, wave, compute, on_start, stamps);
     } else if constexpr (PHASED) {
-      run_k_loop_phased<G>(p, m0, n0, lds, wm, wn, acc, on_start, stamps);
+      run_k_loop_phased<G>(p, m0, n0, lds, wave, wm, wn, acc, on_start, stamps);
     } else {
-      run_k_loop_halves<G, WM>(p, m0, n0, lds, wm, wn, acc, on_start, stamps);
+      run_k_loop_halves<G, WM>(p, m0, n0, lds, wave, wm, wn, acc, on_start, stamps);
     }
     after_k_loop();
 
@@ -630,7 +628,7 @@ struct FmaTile {
   // Multiplies a stage whose first krem values of k lie inside the problem.
   // issue(l) asks for load l of the next stage: one a slice behind its operand
   // reads in the 4 x 4 form, where a lone workgroup has nothing else to hide
-  // them behind (64 problems 1024 to 4096 deep: 193 -> 187 us), else all ahead of
+  // them behind (64 problems 1024 to 4096 deep: 193 -> 181 us), else all ahead of
   // the slices (the larger tiles lose up to 4% with the loads spread out).
   template <class Issue>
   __device__ __forceinline__ static void compute_stage(const uint16_t* stage, int krem, int tm, int tn,
@@ -672,7 +670,7 @@ struct FmaTile {
   // MfmaTile::run.
   template <bool WIDE, class OnStart, class AfterKLoop, class Stamps>
   __device__ __forceinline__ static void run(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
-                                             OnStart&& on_start, AfterKLoop&& after_k_loop, const Stamps& stamps) {
+                                             int wave, OnStart&& on_start, AfterKLoop&& after_k_loop, const Stamps& stamps) {
     const int tid = threadIdx.x;
     const int tm = tid >> 4;
     const int tn = tid & 15;
@@ -716,12 +714,12 @@ struct FmaTile {
 
     if constexpr (WIDE) {
       int kt = 0;
-      run_k_loop<G>(p, m0, n0, lds, [&](const uint16_t* stage) {
+      run_k_loop<G>(p, m0, n0, lds, wave, [&](const uint16_t* stage) {
         if (active) compute_stage(stage, p.k - kt * G::BK, tm, tn, acc, [](int) {});
         ++kt;
       }, on_start, stamps);
     } else {
-      run_k_loop_fma<G>(p, m0, n0, lds, [&](const uint16_t* stage, int k0, auto&& issue) {
+      run_k_loop_fma<G>(p, m0, n0, lds, wave, [&](const uint16_t* stage, int k0, auto&& issue) {
         if (active) {
           compute_stage(stage, p.k - k0, tm, tn, acc, issue);
         } else {
@@ -729,7 +727,7 @@ struct FmaTile {
         }
       }, on_start, stamps);
     }
-    if constexpr (!SMALL) request_c(opaque_tid());
+    if constexpr (!SMALL) request_c(opaque_tid(wave));
     after_k_loop();
 
     if (!active) {
@@ -756,7 +754,7 @@ struct FmaTile {
         }
       }
     } else {
-      const int t = opaque_tid();  // its parts are not held through the k-loop
+      const int t = opaque_tid(wave);  // its parts are not held through the k-loop
       const __amdgpu_buffer_rsrc_t drs =
           buffer_rsrc(p.d + ((int64_t)r0 * p.ldd + n0), 4 * ((int64_t)(p.m - 1 - r0) * p.ldd + (p.n - n0)));
 #pragma unroll
@@ -814,7 +812,7 @@ struct KernelLds<S, true> {
 // class is uniform across the workgroup (scalar descriptor and origin).
 template <class S, int PATH, bool WIDE, class OnStart, class AfterKLoop, class Stamps = NoStamps>
 __device__ __forceinline__ void run_work_tile(const gg_device_problem_desc& p, int m0, int n0,
-                                              StageRing<KernelLds<S>::HALVES>& ring, OnStart&& on_start,
+                                              StageRing<KernelLds<S>::HALVES>& ring, int wave, OnStart&& on_start,
                                               AfterKLoop&& after_k_loop, const Stamps& stamps = Stamps{}) {
   uint16_t* const lds = ring.values;
   if constexpr (PATH == GGK_PATH_MFMA && !WIDE && S::CLASSES) {
@@ -823,16 +821,16 @@ __device__ __forceinline__ void run_work_tile(const gg_device_problem_desc& p, i
     // The full form first: its code then follows the dispatch as it would
     // without the edge classes.
     if (__builtin_expect(!rows && !cols, 1)) {
-      TileFor<S, PATH>::type::template run<false>(p, m0, n0, lds, on_start, after_k_loop, stamps);
+      TileFor<S, PATH>::type::template run<false>(p, m0, n0, lds, wave, on_start, after_k_loop, stamps);
     } else if (!cols) {
-      MfmaTile<typename S::GR, S::WAVE_M_R>::template run<false>(p, m0, n0, lds, on_start, after_k_loop, stamps);
+      MfmaTile<typename S::GR, S::WAVE_M_R>::template run<false>(p, m0, n0, lds, wave, on_start, after_k_loop, stamps);
     } else if (!rows) {
-      MfmaTile<typename S::GC, S::WAVE_M_C>::template run<false>(p, m0, n0, lds, on_start, after_k_loop, stamps);
+      MfmaTile<typename S::GC, S::WAVE_M_C>::template run<false>(p, m0, n0, lds, wave, on_start, after_k_loop, stamps);
     } else {
-      MfmaTile<typename S::GRC, S::WAVE_M_RC>::template run<false>(p, m0, n0, lds, on_start, after_k_loop, stamps);
+      MfmaTile<typename S::GRC, S::WAVE_M_RC>::template run<false>(p, m0, n0, lds, wave, on_start, after_k_loop, stamps);
     }
   } else {
-    TileFor<S, PATH>::type::template run<WIDE>(p, m0, n0, lds, on_start, after_k_loop, stamps);
+    TileFor<S, PATH>::type::template run<WIDE>(p, m0, n0, lds, wave, on_start, after_k_loop, stamps);
   }
 }
 
