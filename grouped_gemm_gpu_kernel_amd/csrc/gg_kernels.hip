@@ -293,9 +293,13 @@ __global__ GG_KERNEL_ATTRS(V, PATH, WIDE) void gg_grouped_kernel(GroupedArgs arg
   // A device-prepared launch of at most half as many work tiles as workgroups
   // (the host does not know how many there are) claims each tile as its two
   // column halves, indices 2 i and 2 i + 1: the other half of the chip would
-  // have nothing to do.  16 experts, 512 tokens, K 1024, N 2048 (120 tiles):
-  // 26.5 -> 21.0 us.  Above half, some workgroups would get two halves, which
-  // cost more than the one tile.
+  // have nothing to do.  Above half, some workgroups would get two halves, which
+  // cost more than the one tile.  On 256 workgroups, whole / in halves (us a pass):
+  //   120 tiles of 100 rows     K 64 21.0 / 19.7, K 1024 32.5 / 28.3, K 4096 69.7 / 58.4
+  //   128 tiles of one row      K 64 18.8 / 17.6, K 1024 30.4 / 26.5, K 4096 65.2 / 55.0
+  //   120 tiles of 100 columns  50.0 / 50.0, 57.4 / 57.4, 79.9 / 80.0 (every second half is empty)
+  //   136 tiles of 200 rows     24.3 / 26.9, 40.4 / 46.8, 97.7 / 131
+  //   248 tiles of 200 rows     31.3 / 35.8, 50.7 / 59.8, 141 / 157
   constexpr bool kSplits = S::CLASSES && !TRACED && !WIDE;
   const int split =
       kSplits && args.header != nullptr && 2 * ((const_int_ptr)args.header)[1] <= grid ? 1 : 0;
