@@ -14,7 +14,6 @@ typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
-typedef float floatx16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 #define GG_LDS __attribute__((address_space(3)))
@@ -47,10 +46,11 @@ constexpr int kStageAlign = 128;
 //      padding.  It flips only chunk-index bits >= 2, so 16-byte pieces
 //      (2 chunks) stay contiguous and every 16-column block stays intact.
 //
-// Register staging: DEPTH stages are in flight in registers at once, the
-// loads of stage k + DEPTH - 1 issued while stage k is multiplied (a ring of
-// DEPTH register sets), written to two LDS buffers.  Loads straight into LDS
-// use BUFFERS LDS buffers, BUFFERS - 1 stages in flight.
+// Stages load straight into BUFFERS LDS buffers; how many of them are in flight
+// is the k-loop's choice.  The 64-bit addressing forms stage through registers
+// instead: DEPTH stages at once, the loads of stage k + DEPTH - 1 issued while
+// stage k is multiplied (a ring of DEPTH register sets), written to two of the
+// LDS buffers.
 template <int BM_, int BN_, int BK_, int DEPTH_, int THREADS_, int BUFFERS_ = 2>
 struct Geometry {
   static constexpr int BM = BM_;

@@ -159,8 +159,8 @@ struct PhasedLoader {
 // wm (128 rows) and block column wn (64 columns); on_start as in the other
 // k-loops.
 template <class G, class OnStart, class Stamps>
-__device__ __forceinline__ void run_k_loop_phased(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds, int wave,
-                                                  int wm, int wn, floatx4_t (&acc)[8][4], OnStart&& on_start,
+__device__ __forceinline__ void run_k_loop_phased(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
+                                                  int wave, int wm, int wn, floatx4_t (&acc)[8][4], OnStart&& on_start,
                                                   const Stamps& stamps) {
   using L = PhasedLoader<G>;
   const int nk = (p.k + G::BK - 1) / G::BK;
@@ -258,7 +258,6 @@ __device__ __forceinline__ void run_k_loop_phased(const gg_device_problem_desc& 
   // one of the last two stages, everything has been issued and the waits count
   // down, the last stage's units being repaired as they land.  LAST: nothing
   // more is read.  The step stamps of a traced launch follow the four phases.
-  const auto nothing = [](int) {};
   auto stage = [&](int kt, auto issue_tag, auto last_tag) {
     constexpr bool ISSUE = decltype(issue_tag)::value, LAST = decltype(last_tag)::value;
     constexpr int N = L::LOADS;

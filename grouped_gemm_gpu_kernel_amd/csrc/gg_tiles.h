@@ -7,8 +7,9 @@
 // K stage is read from global memory into registers while the previous stage,
 // held in LDS, is being multiplied; the registers are then written to the
 // other LDS buffer and one barrier ends the stage.  The reference's
-// equivalents are compute_gemm_tile_tensor_core and compute_gemm_tile_simt (src/grouped_gemm.cu:373-626); the k-loop structure,
-// register blocking and LDS layout here are gfx950's own.
+// equivalents are compute_gemm_tile_tensor_core and compute_gemm_tile_simt
+// (src/grouped_gemm.cu:373-626); the k-loop structure, register blocking and LDS
+// layout here are gfx950's own.
 #pragma once
 
 #include "gg_common.h"
@@ -16,12 +17,12 @@
 
 namespace gg {
 
-// Runs the staged k-loop of one tile in the 64-bit addressing form: compute(stage_pointer) is called once
-// per stage with that stage's LDS buffer, and on_start() once, by every
-// thread, after the first loads are on their way (the persistent scheduler
-// requests its next tile there, so that the request's latency overlaps this
-// tile's).  on_start returns whether the calling wave issued one global
-// memory request of its own.
+// Runs the staged k-loop of one tile in the 64-bit addressing form:
+// compute(stage_pointer) is called once per stage with that stage's LDS buffer,
+// and on_start() once, by every thread, after the first loads are on their way
+// (the persistent scheduler requests its next tile there, so that the request's
+// latency overlaps this tile's).  on_start returns whether the calling wave
+// issued one global memory request of its own.
 //
 // Stage s is fetched into register set s % DEPTH.  While stage k is
 // multiplied out of LDS buffer k % 2, the loads of stage k + DEPTH - 1 are
@@ -94,8 +95,8 @@ __device__ __forceinline__ void run_k_loop(const gg_device_problem_desc& p, int 
 // on_start runs after the first barrier: the request it makes is then the
 // youngest operation in flight, and the first stage's wait lets it stay there.
 template <class G, int WM, class OnStart, class Stamps>
-__device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds, int wave,
-                                                  int wm, int wn, floatx4_t (&acc)[WM / 16][4], OnStart&& on_start,
+__device__ __forceinline__ void run_k_loop_halves(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
+                                                  int wave, int wm, int wn, floatx4_t (&acc)[WM / 16][4], OnStart&& on_start,
                                                   const Stamps& stamps) {
   using L = DmaLoader<G>;
   constexpr int NBUF = G::BUFFERS;
@@ -350,8 +351,9 @@ struct MfmaTile {
   // 140.5.  The 128 x 64 blocks have no registers left for it.
   static constexpr bool EARLY_C = FM <= 4;
 
-  // Multiplies one LDS stage into acc.  All MFMAs of a stage are issued
-  // unconditionally; skipping is decided once per tile for the whole wave.
+  // Multiplies one LDS stage into acc (64-bit addressing form).  All MFMAs of a
+  // stage are issued unconditionally; skipping is decided once per tile for the
+  // whole wave.
   __device__ __forceinline__ static void compute_stage(const uint16_t* stage, int lane, int wm, int wn,
                                                        floatx4_t (&acc)[FM][FN]) {
     const uint16_t* as = stage;
@@ -397,12 +399,17 @@ struct MfmaTile {
   // of this tile follows it: the epilogue works from registers).
   template <bool WIDE, class OnStart, class AfterKLoop, class Stamps>
   __device__ __forceinline__ static void run(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
-                                             int wave, OnStart&& on_start, AfterKLoop&& after_k_loop, const Stamps& stamps) {
+                                             int wave, OnStart&& on_start, AfterKLoop&& after_k_loop,
+                                             const Stamps& stamps) {
     const int lane = opaque_lane();
     const int wm = wave / WAVES_N;
     const int wn = wave % WAVES_N;
-    // A wave whose block starts past the problem's edge has nothing to
-    // multiply or store; it still stages its share of A and B for the others.
+    // A wave whose block starts past the problem's edge has nothing to store; it
+    // still stages its share of A and B for the others.  The pipelined k-loops
+    // multiply for it all the same (their waits and reads are between the MFMAs):
+    // launches of tiles with 1 to 129 rows or 64 to 130 columns, in which up to
+    // seven of eight waves are such, were no slower for it (64 experts of one row,
+    // K = N = 4096: 368 -> 361 us with these loops, of four rows, N 14336: 1269 -> 1264).
     const bool live = m0 + wm * WM < p.m && n0 + wn * WN < p.n;
 
     floatx4_t acc[FM][FN];
@@ -670,7 +677,8 @@ struct FmaTile {
   // MfmaTile::run.
   template <bool WIDE, class OnStart, class AfterKLoop, class Stamps>
   __device__ __forceinline__ static void run(const gg_device_problem_desc& p, int m0, int n0, uint16_t* lds,
-                                             int wave, OnStart&& on_start, AfterKLoop&& after_k_loop, const Stamps& stamps) {
+                                             int wave, OnStart&& on_start, AfterKLoop&& after_k_loop,
+                                             const Stamps& stamps) {
     const int tid = threadIdx.x;
     const int tm = tid >> 4;
     const int tn = tid & 15;
@@ -750,7 +758,8 @@ struct FmaTile {
 #pragma unroll
         for (int j = 0; j < RN; ++j) {
           const int col = n0 + tn * RN + j;
-          if (col < p.n) dptr[(int64_t)row * p.ldd + col] = epilogue_value(acc[i][j], ce[j], p.alpha, use_c ? p.beta : 0.0f);
+          if (col >= p.n) continue;
+          dptr[(int64_t)row * p.ldd + col] = epilogue_value(acc[i][j], ce[j], p.alpha, use_c ? p.beta : 0.0f);
         }
       }
     } else {

@@ -235,11 +235,13 @@ hipError_t ggk_launch_grouped(int variant, int path, int addressing, const gg_de
 /* The same launch, whose completion signals `done` (NULL: no event) when the
  * stream is not capturing; *recorded (may be NULL) as for
  * ggk_event_record_launch.  The signal is the dispatch's own, which costs the
- * stream about 2.5 us less per launch than an event recorded after it. */
+ * stream about 2.5 us less per launch than an event recorded after it; the
+ * runtime keeps the launch's host object until an event recorded on the stream
+ * has been processed, so a caller records one now and then. */
 hipError_t ggk_launch_grouped_done(int variant, int path, int addressing, const gg_device_problem_desc* d_problems,
-                              const int* d_work_offsets, const int* d_order, const int* d_work_table,
-                              int problem_count, int total_work, int* d_state, const int* chunk_bounds, int grid,
-                              hipEvent_t done, int* recorded, hipStream_t stream);
+                                   const int* d_work_offsets, const int* d_order, const int* d_work_table,
+                                   int problem_count, int total_work, int* d_state, const int* chunk_bounds, int grid,
+                                   hipEvent_t done, int* recorded, hipStream_t stream);
 
 /* The same scheduler with instrumentation.  d_tile_map (may be NULL; needs
  * d_tile_offsets, the reference tile offsets of the problems in sorted
@@ -349,9 +351,10 @@ hipError_t ggk_launch_grouped_device(int variant, int path, int addressing, cons
                                      const int* d_work_offsets, const int* d_order, int problem_count,
                                      const int* d_header, int* d_state, int grid, hipStream_t stream);
 /* The same launch, signalling `done` as ggk_launch_grouped_done. */
-hipError_t ggk_launch_grouped_device_done(int variant, int path, int addressing, const gg_device_problem_desc* d_problems,
-                                     const int* d_work_offsets, const int* d_order, int problem_count,
-                                     const int* d_header, int* d_state, int grid, hipEvent_t done, int* recorded, hipStream_t stream);
+hipError_t ggk_launch_grouped_device_done(int variant, int path, int addressing,
+                                          const gg_device_problem_desc* d_problems, const int* d_work_offsets,
+                                          const int* d_order, int problem_count, const int* d_header, int* d_state,
+                                          int grid, hipEvent_t done, int* recorded, hipStream_t stream);
 
 /* One problem, one workgroup per work tile, row-major work-tile order
  * (single_problem_gemm_kernel + launch_single_problem_variant,
