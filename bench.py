@@ -239,9 +239,9 @@ def tile_phases(torch, ex, runs: int = 3) -> dict:
         "all": np.ones(len(ph), bool),
     }
     out = {"work_tiles": int(len(ph)), "work_tile_rows": bm, "work_tile_cols": bn}
-    # The middle k-loop step of each tile, per wave: issuing the next stage's loads, issuing the
-    # MFMAs and fragment reads, the wait for the loads, the closing barrier (mean over the waves),
-    # and the step from the first wave's start to the last wave's barrier.
+    # The middle k-loop step of each tile, per wave: the MFMAs of its first half with the fragment
+    # reads and loads among them, the wait for the next stage's loads, the barrier, the MFMAs of its
+    # second half (mean over the waves), and the step from the first wave's start to the last wave's end.
     step = ph[:, _lib.GGK_PHASE_STEP:].reshape(len(ph), _lib.GGK_PHASE_STEP_WAVES,
                                                 _lib.GGK_PHASE_STEP_MARKS).astype(np.float64)
     stamped = (step[:, :, 0] > 0)
@@ -256,10 +256,10 @@ def tile_phases(torch, ex, runs: int = 3) -> dict:
             w = stamped[st]
             parts = [np.where(w, step[st, :, i + 1] - step[st, :, i], np.nan) for i in range(4)]
             span = (np.where(w, step[st, :, 4], -np.inf).max(axis=1) - np.where(w, step[st, :, 0], np.inf).min(axis=1))
-            step_row = {"issue": round(float(np.nanmean(parts[0]))), "mfma": round(float(np.nanmean(parts[1]))),
-                        "wait": round(float(np.nanmean(parts[2]))), "barrier": round(float(np.nanmean(parts[3]))),
-                        "barrier_max_wave": round(float(np.nanmean(np.nanmax(parts[3], axis=1)))),
-                        "step": round(float(span.mean()))}
+            step_row = {"first_half": round(float(np.nanmean(parts[0]))), "wait": round(float(np.nanmean(parts[1]))),
+                        "barrier": round(float(np.nanmean(parts[2]))),
+                        "barrier_max_wave": round(float(np.nanmean(np.nanmax(parts[2], axis=1)))),
+                        "second_half": round(float(np.nanmean(parts[3]))), "step": round(float(span.mean()))}
             if name == "whole" and bm > 128:
                 step_row = {"phases": [round(float(np.nanmean(x))) for x in parts], "step": round(float(span.mean()))}
         out[name] = {

@@ -265,12 +265,12 @@ enum {
                                  cols << 34 | stages << 46: the tile's rows and columns inside its
                                  problem (at most the work tile's), its k-stages */
   /* Entry GGK_PHASE_STEP + GGK_PHASE_STEP_MARKS w + i: wave w's core clock in the k-loop step
-   * k = stages / 2 (LDS-DMA k-loops only; zero elsewhere): i = 0 the step starts, 1 its loads of
-   * the next stage are issued, 2 its MFMAs and fragment reads are issued, 3 its loads have landed
-   * (the step's vmcnt wait is over), 4 the step's closing barrier is passed.  A work tile with more
-   * than half the rows and half the columns of a 256 x 256 one runs its step in four phases, each
-   * a quarter of the MFMAs, the loads and the fragment reads: there i = 1..4 is the end of phase
-   * i - 1. */
+   * k = stages / 2 (MFMA path with loads straight into LDS; zero elsewhere): i = 0 the step starts,
+   * 1 the MFMAs of its first half, with the fragment reads and loads among them, are issued, 2 the
+   * next stage's loads have landed (the step's vmcnt wait is over), 3 its barrier is passed, 4 the
+   * MFMAs of its second half are issued.  A work tile with more than half the rows and half the
+   * columns of a 256 x 256 one runs its step in four phases, each a quarter of the MFMAs, the loads
+   * and the fragment reads: there i = 1..4 is the end of phase i - 1. */
   GGK_PHASE_STEP = 8,
   GGK_PHASE_STEP_MARKS = 5,
   GGK_PHASE_STEP_WAVES = 8,   /* waves per workgroup at most */
