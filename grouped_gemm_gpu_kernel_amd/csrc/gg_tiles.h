@@ -406,10 +406,10 @@ struct MfmaTile {
     const int wn = wave % WAVES_N;
     // A wave whose block starts past the problem's edge has nothing to store; it
     // still stages its share of A and B for the others.  The pipelined k-loops
-    // multiply for it all the same (their waits and reads are between the MFMAs):
-    // launches of tiles with 1 to 129 rows or 64 to 130 columns, in which up to
-    // seven of eight waves are such, were no slower for it (64 experts of one row,
-    // K = N = 4096: 368 -> 361 us with these loops, of four rows, N 14336: 1269 -> 1264).
+    // multiply for it all the same.  A branch past the MFMAs of such waves took
+    // 64 experts' 1.24 MFMAs per useful one down (2427 -> 2400 us), but breaks up
+    // the interleaving of MFMAs, reads and loads: 24 ragged problems 140.5 -> 143, a
+    // 16-expert layer 29.9 -> 31.2, column-edge tiles 3 to 5% slower.
     const bool live = m0 + wm * WM < p.m && n0 + wn * WN < p.n;
 
     floatx4_t acc[FM][FN];
