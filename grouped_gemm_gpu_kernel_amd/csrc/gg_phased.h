@@ -6,11 +6,12 @@
 // that use them.  With whole stages (all loads of the next stage issued at the
 // top of a step, one stage in flight) the waves spent a third of a step blocked
 // on issuing loads and as much waiting for them: a stage took 4,030 cycles
-// where its MFMAs need 2,048; here it takes 2,900 traced.  Same card: 64 x 2048^3
-// 1221 -> 1005 us, one 8192^3 problem 991 -> 814 us (1350 TFLOP/s).  On random
-// data the clock falls to 1.9 GHz and below under the chip's power limit (zeros:
-// 609 us at 2.4 GHz), so what bounds the loop is energy per product: without
-// its loads it takes 16% less time, without its fragment reads 17%.
+// where its MFMAs need 2,048; here it takes 2,900 to 3,100 traced.  Same card: 64 x
+// 2048^3 1221 -> 1005 us, one 8192^3 problem 991 -> 814 us (1350 TFLOP/s).  On random
+// data the clock falls to 1.7 GHz under the chip's power limit (zeros: 595 us at 2.4
+// GHz, with the same 73% of the SIMDs' cycles in MFMAs), so what bounds the loop is
+// energy per product: without its loads it takes 16% less time, without its
+// fragment reads 17%.
 #pragma once
 
 #include <type_traits>
